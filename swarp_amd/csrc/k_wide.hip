@@ -6,8 +6,8 @@
 namespace swarp {
 template void launch_wide_lists<SWARP_T>(const Cst<SWARP_T> &, const SWARP_T *, const SWARP_T *,
                                          int32_t *, int32_t *, int32_t *, hipStream_t);
-template void launch_grid_frame<SWARP_T>(const SWARP_T *, int64_t, SWARP_T, int, SWARP_T *,
-                                         hipStream_t);
+template void launch_grid_frame<SWARP_T>(const SWARP_T *, int64_t, SWARP_T, int, void *, uint64_t,
+                                         SWARP_T *, hipStream_t);
 template void launch_wide_fwd_apt<SWARP_T, 1>(bool, bool, const Cst<SWARP_T> &,
                                               const Args<SWARP_T> &, hipStream_t);
 template void launch_wide_bwd_apt<SWARP_T, 1>(bool, bool, const Cst<SWARP_T> &,

@@ -43,7 +43,8 @@
                                              int32_t *, int32_t *, hipStream_t);             \
     extern template void launch_wide_lists<T>(const Cst<T> &, const T *, const T *, int32_t *,\
                                               int32_t *, int32_t *, hipStream_t);            \
-    extern template void launch_grid_frame<T>(const T *, int64_t, T, int, T *, hipStream_t);  \
+    extern template void launch_grid_frame<T>(const T *, int64_t, T, int, void *, uint64_t,   \
+                                              T *, hipStream_t);                             \
     extern template void launch_wide_fwd_apt<T, 1>(bool, bool, const Cst<T> &, const Args<T> &, \
                                                    hipStream_t);                             \
     extern template void launch_wide_fwd_apt<T, 2>(bool, bool, const Cst<T> &, const Args<T> &, \

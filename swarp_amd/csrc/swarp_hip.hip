@@ -937,6 +937,7 @@ int swarp_neighbors(const swarp_desc_t *desc, const void *pos, int32_t *idx, int
     const int PA = pad_agents(desc->n_agents);
     const bool adaptive = desc->neighbor_method == SWARP_LISTS_GRID && !desc->grid_pinned;
     if (adaptive && !desc->grid_frame) return fail("grid_frame must be set for an adaptive grid frame");
+    const uint64_t list_bytes = (uint64_t)desc->n_envs * desc->n_agents * desc->max_neighbors * 4;
     if (desc->dtype == SWARP_F32) {
         if (wide_path(desc) && wide_lds_check<float>(desc, true)) return -1;
         Cst<float> C;
@@ -945,7 +946,7 @@ int swarp_neighbors(const swarp_desc_t *desc, const void *pos, int32_t *idx, int
             float *fr = adaptive ? (float *)desc->grid_frame : nullptr;
             if (adaptive)
                 launch_grid_frame<float>((const float *)pos, (int64_t)C.E * C.A,
-                                         (float)desc->neighbor_radius, C.grid_bins, fr, st);
+                                         (float)desc->neighbor_radius, C.grid_bins, idx, list_bytes, fr, st);
             launch_wide_lists<float>(C, (const float *)pos, fr, idx, cnt, true_cnt, st);
         } else {
             launch_neighbors<float>(PA, C, (const float *)pos, idx, cnt, true_cnt, st);
@@ -958,7 +959,7 @@ int swarp_neighbors(const swarp_desc_t *desc, const void *pos, int32_t *idx, int
             double *fr = adaptive ? (double *)desc->grid_frame : nullptr;
             if (adaptive)
                 launch_grid_frame<double>((const double *)pos, (int64_t)C.E * C.A,
-                                          desc->neighbor_radius, C.grid_bins, fr, st);
+                                          desc->neighbor_radius, C.grid_bins, idx, list_bytes, fr, st);
             launch_wide_lists<double>(C, (const double *)pos, fr, idx, cnt, true_cnt, st);
         } else {
             launch_neighbors<double>(PA, C, (const double *)pos, idx, cnt, true_cnt, st);

@@ -154,6 +154,13 @@ __device__ inline void block_exclusive_scan(int32_t *v, int n, int32_t *wsum)
 // smaller index), cstart[c] (first sorted slot of cell c, cstart[NC] = A), sorted[]
 // (agent indices cell by cell, ascending within a cell).  The
 // positions are in W.px / W.py.  Every thread of the workgroup calls it.
+//
+// A counting sort whose ranks cost an agent its own cell's occupants (about one at the
+// default bins) instead of a pass over all smaller indices: the counting atomics hand every
+// agent a slot of its cell in arrival order, the agent counts its cell's members of smaller
+// index there, and the second scatter puts the cell in index order.  The O(A) pass bound
+// the list build: 200 envs x 1000 agents 45 -> 30 us, and at 48 x 2000 agents the forward
+// rollout of 8 steps x 2 substeps 3.16 -> 0.52 ms, its backward 5.20 -> 1.40 ms.
 template <typename T>
 __device__ inline void grid_build(const WideLds<T> &W, int A, const GridFrame<T> &G,
                                   int32_t *wsum)
@@ -166,17 +173,20 @@ __device__ inline void grid_build(const WideLds<T> &W, int A, const GridFrame<T>
         const int cy = grid_axis(W.py[i], G.oy, G.cs, G.bins);
         const int k = cy * G.bins + cx;
         W.key[i] = k;
-        atomicAdd(&W.cstart[k], 1);
+        W.rank[i] = atomicAdd(&W.cstart[k], 1);  // arrival slot: the rank in any order
     }
     __syncthreads();
     block_exclusive_scan(W.cstart, NC, wsum);
+    for (int i = tid; i < A; i += nt) W.sorted[W.cstart[W.key[i]] + W.rank[i]] = i;
+    __syncthreads();
     for (int i = tid; i < A; i += nt) {
-        const int k = W.key[i];
-        int r = 0;  // agents of the same cell with a smaller index
-        for (int j = 0; j < i; ++j) r += W.key[j] == k ? 1 : 0;
+        const int k = W.key[i], c1 = W.cstart[k + 1];
+        int r = 0;
+        for (int q = W.cstart[k]; q < c1; ++q) r += W.sorted[q] < i ? 1 : 0;
         W.rank[i] = r;
-        W.sorted[W.cstart[k] + r] = i;
     }
+    __syncthreads();
+    for (int i = tid; i < A; i += nt) W.sorted[W.cstart[W.key[i]] + W.rank[i]] = i;
     __syncthreads();
 }
 
@@ -264,50 +274,98 @@ __device__ __forceinline__ GridFrame<T> grid_frame(const Cst<T> &C, const T *fra
 
 // _bounds_init / _bounds_reduce / _finalize_grid (swarp/core/neighbors.py:149-181): the
 // batch's min corner, extent max(dx, dy), cell size max(radius, extent / bins), in T.
-template <typename T>
-__global__ __launch_bounds__(1024) void k_grid_frame(const T *pos, int64_t n, T radius, int bins,
-                                                     T *frame)
+//
+// Two launches above FRAME_ONE positions: FRAME_BLOCK positions to a workgroup, each
+// leaving its box (min x, min y, max x, max y) in `part`, then one workgroup over the
+// boxes.  One workgroup over all positions was latency bound on one CU: 66 us for 200000
+// agents against 4.9 + 1.9 us.  Up to FRAME_ONE positions one workgroup takes them all (8
+// rounds of loads a lane: no slower than a second launch).  Minima and maxima do not depend
+// on the order.
+constexpr int64_t FRAME_BLOCK = 2048, FRAME_ONE = 2048;
+
+template <typename T> struct Box4 {
+    T mnx, mny, mxx, mxy;
+};
+
+template <typename T> __device__ __forceinline__ void box_join(Box4<T> &a, const Box4<T> &b)
 {
-    __shared__ T red[4][16];
-    const T big = T(1e30);
-    T mnx = big, mny = big, mxx = -big, mxy = -big;
-    for (int64_t q = threadIdx.x; q < n; q += 1024) {
-        const T x = pos[2 * q], y = pos[2 * q + 1];
-        mnx = x < mnx ? x : mnx;
-        mny = y < mny ? y : mny;
-        mxx = x > mxx ? x : mxx;
-        mxy = y > mxy ? y : mxy;
-    }
-    for (int d = 32; d > 0; d >>= 1) {
-        const T a = __shfl_down(mnx, d, 64), b = __shfl_down(mny, d, 64);
-        const T c = __shfl_down(mxx, d, 64), e = __shfl_down(mxy, d, 64);
-        mnx = a < mnx ? a : mnx;
-        mny = b < mny ? b : mny;
-        mxx = c > mxx ? c : mxx;
-        mxy = e > mxy ? e : mxy;
-    }
+    a.mnx = b.mnx < a.mnx ? b.mnx : a.mnx;
+    a.mny = b.mny < a.mny ? b.mny : a.mny;
+    a.mxx = b.mxx > a.mxx ? b.mxx : a.mxx;
+    a.mxy = b.mxy > a.mxy ? b.mxy : a.mxy;
+}
+
+template <typename T> __device__ __forceinline__ Box4<T> box_none()
+{
+    return {T(1e30), T(1e30), T(-1e30), T(-1e30)};
+}
+
+// The workgroup's box (256 threads) in thread 0.
+template <typename T> __device__ __forceinline__ void box_reduce(Box4<T> &m, T (&red)[4][4])
+{
+    for (int d = 32; d > 0; d >>= 1)
+        box_join(m, Box4<T>{__shfl_down(m.mnx, d, 64), __shfl_down(m.mny, d, 64),
+                            __shfl_down(m.mxx, d, 64), __shfl_down(m.mxy, d, 64)});
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     if (lane == 0) {
-        red[0][wv] = mnx;
-        red[1][wv] = mny;
-        red[2][wv] = mxx;
-        red[3][wv] = mxy;
+        red[wv][0] = m.mnx;
+        red[wv][1] = m.mny;
+        red[wv][2] = m.mxx;
+        red[wv][3] = m.mxy;
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int w = 1; w < 16; ++w) {
-            mnx = red[0][w] < mnx ? red[0][w] : mnx;
-            mny = red[1][w] < mny ? red[1][w] : mny;
-            mxx = red[2][w] > mxx ? red[2][w] : mxx;
-            mxy = red[3][w] > mxy ? red[3][w] : mxy;
-        }
-        const T ex = mxx - mnx, ey = mxy - mny;
-        const T ext = ex > ey ? ex : ey;
-        const T q = ext / T(bins);
-        frame[0] = mnx;
-        frame[1] = mny;
-        frame[2] = radius > q ? radius : q;
+    if (threadIdx.x == 0)
+        for (int w = 1; w < 4; ++w)
+            box_join(m, Box4<T>{red[w][0], red[w][1], red[w][2], red[w][3]});
+}
+
+template <typename T>
+__device__ __forceinline__ void frame_put(const Box4<T> &m, T radius, int bins, T *frame)
+{
+    const T ex = m.mxx - m.mnx, ey = m.mxy - m.mny;
+    const T ext = ex > ey ? ex : ey;
+    const T q = ext / T(bins);
+    frame[0] = m.mnx;
+    frame[1] = m.mny;
+    frame[2] = radius > q ? radius : q;
+}
+
+// The boxes of `per` positions a workgroup into `part`, or (ONE, one workgroup) the frame.
+template <typename T, bool ONE>
+__global__ __launch_bounds__(256) void k_frame_boxes(const T *pos, int64_t n, int64_t per, T *part,
+                                                     T radius, int bins, T *frame)
+{
+    __shared__ T red[4][4];
+    Box4<T> m = box_none<T>();
+    const int64_t q0 = (int64_t)blockIdx.x * per;
+    const int64_t q1 = q0 + per < n ? q0 + per : n;
+    for (int64_t q = q0 + threadIdx.x; q < q1; q += 256) {
+        const T x = pos[2 * q], y = pos[2 * q + 1];
+        box_join(m, Box4<T>{x, y, x, y});
     }
+    box_reduce(m, red);
+    if (threadIdx.x != 0) return;
+    if (ONE) {
+        frame_put(m, radius, bins, frame);
+    } else {
+        T *o = part + 4 * (int64_t)blockIdx.x;
+        o[0] = m.mnx;
+        o[1] = m.mny;
+        o[2] = m.mxx;
+        o[3] = m.mxy;
+    }
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void k_grid_frame(const T *part, int64_t n, T radius, int bins,
+                                                    T *frame)
+{
+    __shared__ T red[4][4];
+    Box4<T> m = box_none<T>();
+    for (int64_t q = threadIdx.x; q < n; q += 256)
+        box_join(m, Box4<T>{part[4 * q], part[4 * q + 1], part[4 * q + 2], part[4 * q + 3]});
+    box_reduce(m, red);
+    if (threadIdx.x == 0) frame_put(m, radius, bins, frame);
 }
 
 // ------------------------------------------------------------------ neighbour lists
@@ -852,10 +910,25 @@ void launch_wide_lists(const Cst<T> &C, const T *pos, const T *frame, int32_t *i
         hipLaunchKernelGGL((k_wide_lists<T, false>), grid, block, shm, st, C, pos, frame, idx, cnt, tru);
 }
 
+// `scratch`: device memory the two-launch reduction may overwrite (the list buffer the
+// build fills afterwards), `bytes` long; too little of it, or not aligned for T, and one
+// workgroup reduces every position.
 template <typename T>
-void launch_grid_frame(const T *pos, int64_t n, T radius, int bins, T *frame, hipStream_t st)
+void launch_grid_frame(const T *pos, int64_t n, T radius, int bins, void *scratch, uint64_t bytes,
+                       T *frame, hipStream_t st)
 {
-    hipLaunchKernelGGL((k_grid_frame<T>), dim3(1), dim3(1024), 0, st, pos, n, radius, bins, frame);
+    const int64_t nb = (n + FRAME_BLOCK - 1) / FRAME_BLOCK;
+    T *part = (T *)scratch;
+    if (n <= FRAME_ONE || bytes < (uint64_t)nb * 4 * sizeof(T) ||
+        (uintptr_t)scratch % sizeof(T) != 0) {
+        hipLaunchKernelGGL((k_frame_boxes<T, true>), dim3(1), dim3(256), 0, st, pos, n, n, part,
+                           radius, bins, frame);
+        return;
+    }
+    hipLaunchKernelGGL((k_frame_boxes<T, false>), dim3((unsigned)nb), dim3(256), 0, st, pos, n,
+                       FRAME_BLOCK, part, radius, bins, frame);
+    hipLaunchKernelGGL((k_grid_frame<T>), dim3(1), dim3(256), 0, st, (const T *)part, nb, radius,
+                       bins, frame);
 }
 
 // boxes: a box world (box agents or wheel contacts; never with drones).
