@@ -82,8 +82,8 @@ template <typename T> struct Args {
     int nsteps;
     // Force tape (nullable): per step, substep and agent the total force the forward
     // integrated (listed pairs, static obstacles, walls), [T][S][E A] pairs -- written by
-    // the generic forward kernels (worlds without box agents or wheel contacts), read by
-    // the backward's recompute in place of evaluating the forces again.
+    // the generic and wide forward kernels (worlds without box agents or wheel contacts),
+    // read by the backward's recompute in place of evaluating the forces again.
     T *fsum;
     // Obstacle-contact tape (nullable, with fsum, at most 32 obstacles): per step, substep
     // and agent a mask of the obstacles whose narrow phase took its contact branch, bit o
@@ -96,6 +96,10 @@ template <typename T> struct Args {
     // agent contacts), written with fsum -- the backward's recompute reads it instead of
     // scanning.
     void *nmask;
+    // Touch tape of the wide kernels (nullable, with fsum; worlds with agent contacts): per
+    // step, substep and agent the agents it touched, [T][S][E A] words of four 16-bit ids
+    // (NearRec); touch2 is written only where touch holds four.
+    uint64_t *touch, *touch2;
 };
 
 // Width of one obstacle-contact mask word for N obstacles (0: no mask above 32).

@@ -6,7 +6,7 @@
 #include "bodies.hpp"
 #include "nav.hpp"
 #include "neighbors.hpp"
-#include "wide.hpp"
+#include "swarm.hpp"
 #include "wide_bodies.hpp"
 
 #define SWARP_EXTERN_LAUNCHERS(T)                                                            \
@@ -46,17 +46,17 @@
     extern template void launch_grid_frame<T>(const T *, int64_t, T, int, void *, uint64_t,   \
                                               T *, hipStream_t);                             \
     extern template void launch_wide_fwd_apt<T, 1>(bool, bool, const Cst<T> &, const Args<T> &, \
-                                                   hipStream_t);                             \
+                                                   unsigned, hipStream_t);                   \
     extern template void launch_wide_fwd_apt<T, 2>(bool, bool, const Cst<T> &, const Args<T> &, \
-                                                   hipStream_t);                             \
+                                                   unsigned, hipStream_t);                   \
     extern template void launch_wide_fwd_apt<T, 4>(bool, bool, const Cst<T> &, const Args<T> &, \
-                                                   hipStream_t);                             \
+                                                   unsigned, hipStream_t);                   \
     extern template void launch_wide_bwd_apt<T, 1>(bool, bool, const Cst<T> &, const Args<T> &, \
-                                                   hipStream_t);                             \
+                                                   unsigned, hipStream_t);                   \
     extern template void launch_wide_bwd_apt<T, 2>(bool, bool, const Cst<T> &, const Args<T> &, \
-                                                   hipStream_t);                             \
+                                                   unsigned, hipStream_t);                   \
     extern template void launch_wide_bwd_apt<T, 4>(bool, bool, const Cst<T> &, const Args<T> &, \
-                                                   hipStream_t);                             \
+                                                   unsigned, hipStream_t);                   \
     extern template void launch_wbody_fwd<T>(bool, const Cst<T> &, const Args<T> &,           \
                                              const ObTab<T> &, const ObIO<T> &, hipStream_t); \
     extern template void launch_wbody_bwd<T>(bool, const Cst<T> &, const Args<T> &,           \

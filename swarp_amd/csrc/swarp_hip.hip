@@ -162,12 +162,24 @@ static int pad_agents(int A)
     return p;
 }
 
+// The wide-env kernels (one workgroup per env): more than 64 agents, or grid-ordered lists.
+static bool wide_path(const swarp_desc_t *d)
+{
+    return d->n_agents > 64 || d->neighbor_method == SWARP_LISTS_GRID;
+}
+
 static double skin_of(const swarp_desc_t *d)
 {
     // Candidate-list skin: room for (S-1) substeps of motion of both agents of a pair
     // at about 1.5x the fleet's top speed.  Only speed depends on it; exactness does not.
-    if (d->substeps < 2) return 0.0;
     const double vmax = d->skin_speed > 0.0 ? d->skin_speed : 1.0;
+    // The wide disc kernels keep candidates across steps: about two steps of motion, at most
+    // two neighbour radii (a wider skin costs a longer list for few searches saved).
+    if (wide_path(d)) {
+        const double two = 2.0 * 2.2 * vmax * d->dt, most = 2.0 * d->neighbor_radius;
+        return two < most ? two : most;
+    }
+    if (d->substeps < 2) return 0.0;
     return 2.0 * 1.5 * vmax * (d->substeps - 1) * (d->dt / d->substeps);
 }
 
@@ -229,12 +241,6 @@ static unsigned world_features(const swarp_desc_t *d, bool body)
     return f;
 }
 
-// The wide-env kernels (one workgroup per env): more than 64 agents, or grid-ordered lists.
-static bool wide_path(const swarp_desc_t *d)
-{
-    return d->n_agents > 64 || d->neighbor_method == SWARP_LISTS_GRID;
-}
-
 // What the wide-env kernels do not step, as an error message (NULL: they step it).
 static const char *wide_unsupported(const swarp_desc_t *d)
 {
@@ -274,9 +280,10 @@ static bool lean_ok(const swarp_desc_t *d)
 // 2-D fleets among static obstacles keeps each substep's total forces (fsum, read by the
 // backward's recompute), each substep's neighbour-inclusion masks (nmask, read by the
 // recompute in place of its scan) and, for at most 32 obstacles, each substep's obstacle
-// contact masks (omask, read by its reverse pass).
+// contact masks (omask, read by its reverse pass).  The wide disc kernels keep each substep's
+// total forces and the agents each agent touched (touch, touch2).
 struct TapeLayout {
-    uint64_t rec, vl, fsum, omask, nmask, total;
+    uint64_t rec, vl, fsum, omask, nmask, touch, touch2, total;
 };
 
 static uint64_t align256(uint64_t x) { return (x + 255) & ~(uint64_t)255; }
@@ -311,9 +318,27 @@ static bool gen_tape_ok(const swarp_desc_t *d)
            (d->collisions || d->soft_walls || d->n_obstacles > 0);
 }
 
+// Whether the wide disc kernels keep a tape, and up to what size (beyond it the backward
+// recomputes: 24 bytes per agent and substep in float32 against the trajectory's 28 per step).
+constexpr uint64_t WIDE_TAPE_MAX = 16ull << 30;
+static bool wide_tape_ok(const swarp_desc_t *d)
+{
+    return wide_path(d) && !d->has_boxes && !d->wheel_contacts &&
+           (d->collisions || d->soft_walls || d->n_obstacles > 0);
+}
+
 static TapeLayout tape_layout(const swarp_desc_t *d, int32_t nT)
 {
-    TapeLayout L = {0, 0, 0, 0, 0, 0};
+    TapeLayout L = {0, 0, 0, 0, 0, 0, 0, 0};
+    if (nT >= 1 && wide_tape_ok(d)) {
+        const uint64_t n = (uint64_t)nT * d->substeps * d->n_envs * d->n_agents;
+        const uint64_t ids = d->collisions ? n * sizeof(uint64_t) : 0;
+        L.touch = align256(n * 2 * (d->dtype == SWARP_F32 ? 4 : 8));
+        L.touch2 = align256(L.touch + ids);
+        L.total = align256(L.touch2 + ids);
+        if (L.total > WIDE_TAPE_MAX) L.total = 0;
+        return L;
+    }
     if (nT >= 1 && split_ok(d)) {
         const uint64_t n = (uint64_t)nT * d->substeps * d->n_envs * d->n_agents;
         L.fsum = 0;
@@ -353,6 +378,16 @@ template <typename T> static Tape<T> tape_ptrs(const TapeLayout &L, void *base)
 }
 
 template <typename T>
+static void wide_tape_ptrs(const swarp_desc_t *d, const TapeLayout &L, const void *base, Args<T> &a)
+{
+    if (!base || !L.total || !wide_tape_ok(d)) return;
+    unsigned char *b = (unsigned char *)base;
+    a.fsum = (T *)b;
+    a.touch = (uint64_t *)(b + L.touch);
+    a.touch2 = (uint64_t *)(b + L.touch2);
+}
+
+template <typename T>
 static int rollout_fwd(const swarp_desc_t *d, int32_t nT, const swarp_state_t *s0,
                        const void *act, const swarp_state_t *traj, const swarp_state_t *fin,
                        void *tape, uint64_t tape_bytes, hipStream_t st)
@@ -378,12 +413,13 @@ static int rollout_fwd(const swarp_desc_t *d, int32_t nT, const swarp_state_t *s
         if (split_ok(d) && omask_bytes(d->n_obstacles)) a.omask = (unsigned char *)tape + TL.omask;
         a.nmask = (unsigned char *)tape + TL.nmask;
     }
+    wide_tape_ptrs(d, TL, tape, a);
     const int PA = pad_agents(d->n_agents);
     const unsigned feat = world_features(d, false);
     if (wide_path(d)) {
         if (const char *why = wide_unsupported(d)) return fail(why);
         if (wide_lds_check<T>(d)) return -1;
-        launch_wide_fwd<T>(d->has_drone != 0, d->has_boxes || d->wheel_contacts, C, a, st);
+        launch_wide_fwd<T>(d->has_drone != 0, d->has_boxes || d->wheel_contacts, C, a, feat, st);
     } else if (lean_ok(d)) {
         if (tape && TL.total)
             launch_holo_fwd<T, true>(PA, C, a, tape_ptrs<T>(TL, tape), st);
@@ -430,11 +466,12 @@ static int rollout_bwd(const swarp_desc_t *d, int32_t nT, const swarp_state_t *s
         if (split_ok(d) && omask_bytes(d->n_obstacles)) a.omask = (unsigned char *)tape + TL.omask;
         a.nmask = (unsigned char *)tape + TL.nmask;
     }
+    wide_tape_ptrs(d, TL, tape, a);
     const int PA = pad_agents(d->n_agents);
     if (wide_path(d)) {
         if (const char *why = wide_unsupported(d)) return fail(why);
         if (wide_lds_check<T>(d)) return -1;
-        launch_wide_bwd<T>(d->has_drone != 0, d->has_boxes != 0, C, a, st);
+        launch_wide_bwd<T>(d->has_drone != 0, d->has_boxes != 0, C, a, world_features(d, false), st);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return fail(hipGetErrorString(e));
         return 0;

@@ -7,7 +7,8 @@
 // radii in LDS.  They serve every 2-D or drone fleet (any model, control mode, obstacles,
 // walls, clamp, integrator, box agents, wheel contacts) of more than 64 agents per env,
 // and every fleet whose lists follow the uniform grid, as far as the env's staging fits
-// the 160 KiB of LDS of a workgroup.
+// the 160 KiB of LDS of a workgroup.  Here: the layout, the list traversals, the list build
+// and the rollouts of box worlds; swarm.hpp rolls out the disc fleets.
 //
 // List order (which K in-radius neighbours a capped list keeps, and the order the pair
 // forces are summed in):
@@ -25,9 +26,9 @@
 // backward gathers each pair's two sides with that test, as the generic kernels do with
 // their masks.
 //
-// The backward recomputes, for each substep in reverse, the substeps before it from the
-// step's checkpoint (S (S + 1) / 2 forward substeps per step): no per-substep state of
-// the env has to fit in LDS.
+// A backward without a tape recomputes, for each substep in reverse, the substeps before it
+// from the step's checkpoint (S (S + 1) / 2 forward substeps per step): no per-substep state
+// of the env has to fit in LDS.
 //
 // Box worlds (BOXES: some agent is a box, or wheel contacts) also stage each agent's
 // heading, spin and heading cos / sin per substep and its footprint per launch (WBoxLds):
@@ -140,7 +141,6 @@ __device__ inline void block_exclusive_scan(int32_t *v, int n, int32_t *wsum)
     int32_t before = 0;
     for (int w = 0; w < wv; ++w) before += wsum[w];
     int32_t run = before + x - s;
-    __syncthreads();
     for (int c = lo; c < hi; ++c) {
         const int32_t t = v[c];
         v[c] = run;
@@ -159,8 +159,8 @@ __device__ inline void block_exclusive_scan(int32_t *v, int n, int32_t *wsum)
 // default bins) instead of a pass over all smaller indices: the counting atomics hand every
 // agent a slot of its cell in arrival order, the agent counts its cell's members of smaller
 // index there, and the second scatter puts the cell in index order.  The O(A) pass bound
-// the list build: 200 envs x 1000 agents 45 -> 30 us, and at 48 x 2000 agents the forward
-// rollout of 8 steps x 2 substeps 3.16 -> 0.52 ms, its backward 5.20 -> 1.40 ms.
+// the list build (200 envs x 1000 agents: 45 -> 30 us) and every kernel that sorts at each
+// substep (48 x 2000 agents, 8 steps of 2 substeps: forward 3.16 -> 0.52 ms).
 template <typename T>
 __device__ inline void grid_build(const WideLds<T> &W, int A, const GridFrame<T> &G,
                                   int32_t *wsum)
@@ -300,12 +300,18 @@ template <typename T> __device__ __forceinline__ Box4<T> box_none()
     return {T(1e30), T(1e30), T(-1e30), T(-1e30)};
 }
 
-// The workgroup's box (256 threads) in thread 0.
-template <typename T> __device__ __forceinline__ void box_reduce(Box4<T> &m, T (&red)[4][4])
+// The wave's box in its first lane.
+template <typename T> __device__ __forceinline__ void box_wave(Box4<T> &m)
 {
     for (int d = 32; d > 0; d >>= 1)
         box_join(m, Box4<T>{__shfl_down(m.mnx, d, 64), __shfl_down(m.mny, d, 64),
                             __shfl_down(m.mxx, d, 64), __shfl_down(m.mxy, d, 64)});
+}
+
+// The workgroup's box (256 threads) in thread 0.
+template <typename T> __device__ __forceinline__ void box_reduce(Box4<T> &m, T (&red)[4][4])
+{
+    box_wave(m);
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     if (lane == 0) {
         red[wv][0] = m.mnx;
@@ -457,6 +463,19 @@ __device__ __forceinline__ void wide_publish(const Cst<T> &C, const WideLds<T> &
     if (GRID && C.collisions) grid_build(W, C.A, G, wsum);
 }
 
+// The same for the APT agents of each thread.
+template <typename T, bool GRID, int APT>
+__device__ __forceinline__ void wide_publish_all(const Cst<T> &C, const WideLds<T> &W,
+                                                 const GridFrame<T> &G, const WLane<T> (&L)[APT],
+                                                 const St<T> (&st)[APT], int32_t *wsum)
+{
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < APT; ++k) wide_put(W, L[k], st[k], (const WBoxLds<T> *)nullptr);
+    __syncthreads();
+    if (GRID) grid_build(W, C.A, G, wsum);
+}
+
 // Contact and static forces of the lane's agent (collision_forces_kernel, swarp/core/
 // collisions.py:818-881: listed pairs in list order, then obstacles, then walls); `cut`
 // receives the key of the K-th listed neighbour (CUT_ALL when the list is not full).
@@ -499,21 +518,51 @@ __device__ __forceinline__ void wide_forces_with(const Cst<T> &C, const WideLds<
     Fy = fy + sy;
 }
 
+// The static obstacles' forces on the lane's agent, in index order.
+template <typename T>
+__device__ __forceinline__ void wide_obstacles(const Cst<T> &C, const Args<T> &g, const WLane<T> &L,
+                                               const St<T> &st, T &sx, T &sy)
+{
+    const size_t eN = (size_t)L.env * C.N;
+    for (int o = 0; o < C.N; ++o) {
+        T gx, gy;
+        obstacle_force(C, g.obs, eN, o, st.px, st.py, st.vx, st.vy, L.pr.radius, L.ddv, gx, gy);
+        sx += gx;
+        sy += gy;
+    }
+}
+
+template <typename T>
+__device__ __forceinline__ void wide_walls(const Cst<T> &C, const WLane<T> &L, const St<T> &st,
+                                           T &sx, T &sy)
+{
+    if (!C.soft_walls) return;
+    T gx, gy;
+    unsigned wb;
+    wall_force_axes(C, st.px, st.py, st.vx, st.vy, L.pr.radius, L.ddv, gx, gy, wb);
+    sx += gx;
+    sy += gy;
+}
+
+// Obstacles, then walls: the part of a substep's force that needs no other agent.
+template <typename T>
+__device__ __forceinline__ void wide_static_forces(const Cst<T> &C, const Args<T> &g,
+                                                   const WLane<T> &L, const St<T> &st, T &sx, T &sy)
+{
+    sx = T(0);
+    sy = T(0);
+    if (L.active) wide_obstacles(C, g, L, st, sx, sy);
+    wide_walls(C, L, st, sx, sy);
+}
+
 template <typename T, bool GRID>
 __device__ __forceinline__ void wide_forces(const Cst<T> &C, const Args<T> &g,
                                             const WideLds<T> &W, const GridFrame<T> &G,
                                             const WLane<T> &L, const St<T> &st, T &Fx, T &Fy,
                                             int32_t &cut)
 {
-    wide_forces_with<T, GRID>(C, W, G, L, st, Fx, Fy, cut, [&](T &sx, T &sy) {
-        const size_t eN = (size_t)L.env * C.N;
-        for (int o = 0; o < C.N; ++o) {
-            T gx, gy;
-            obstacle_force(C, g.obs, eN, o, st.px, st.py, st.vx, st.vy, L.pr.radius, L.ddv, gx, gy);
-            sx += gx;
-            sy += gy;
-        }
-    });
+    wide_forces_with<T, GRID>(C, W, G, L, st, Fx, Fy, cut,
+                              [&](T &sx, T &sy) { wide_obstacles(C, g, L, st, sx, sy); });
 }
 
 // The forces of a box world (collision_forces_box_kernel, swarp/core/collisions.py:
@@ -699,7 +748,8 @@ __device__ __forceinline__ void wide_lanes(const Cst<T> &C, const Args<T> &g, co
     }
 }
 
-template <typename T, bool DRONE, bool GRID, bool BOXES, int APT, unsigned F>
+// The forward rollout of box worlds (the disc fleets' kernels are swarm.hpp's).
+template <typename T, bool GRID, int APT, unsigned F>
 __global__ __launch_bounds__(1024) void k_wide_fwd(const Cst<T> Cin, const Args<T> g)
 {
     const Cst<T> C = fold_cst<F>(Cin);
@@ -710,26 +760,40 @@ __global__ __launch_bounds__(1024) void k_wide_fwd(const Cst<T> Cin, const Args<
     const WBoxLds<T> B = wide_box_lds<T>(smem, AP, wide_cells(C));
     const GridFrame<T> G = grid_frame(C, (const T *)nullptr);
     WLane<T> L[APT];
-    wide_lanes<T, BOXES, APT, F>(C, g, W, B, L);
+    wide_lanes<T, true, APT, F>(C, g, W, B, L);
     St<T> st[APT];
 #pragma unroll
-    for (int k = 0; k < APT; ++k) load_state<T, DRONE>(g.s0.f, L[k].idx, 0, st[k]);
+    for (int k = 0; k < APT; ++k) load_state<T, false>(g.s0.f, L[k].idx, 0, st[k]);
     const size_t EA = (size_t)C.E * C.A;
     for (int t = 0; t < g.nsteps; ++t) {
         T a[APT][4];
 #pragma unroll
         for (int k = 0; k < APT; ++k) load_act(g.act, (size_t)t * EA + L[k].idx, C.ad, a[k]);
         for (int s = 0; s < C.S; ++s)
-            wide_substep<T, DRONE, GRID, BOXES, APT>(C, g, W, B, G, L, a, st, wsum);
+            wide_substep<T, false, GRID, true, APT>(C, g, W, B, G, L, a, st, wsum);
 #pragma unroll
         for (int k = 0; k < APT; ++k) {
             if (!L[k].active) continue;
             if (t + 1 < g.nsteps)
-                store_state<T, DRONE>(g.traj.f, (size_t)t * EA + L[k].idx, st[k]);
+                store_state<T, false>(g.traj.f, (size_t)t * EA + L[k].idx, st[k]);
             else
-                store_state<T, DRONE>(g.fin.f, L[k].idx, st[k]);
+                store_state<T, false>(g.fin.f, L[k].idx, st[k]);
         }
     }
+}
+
+// Reverse of wide_static_forces.
+template <typename T>
+__device__ __forceinline__ void wide_static_adj(const Cst<T> &C, const Args<T> &g,
+                                                const WLane<T> &L, const St<T> &in, T gFx, T gFy,
+                                                St<T> &gi)
+{
+    const size_t eN = (size_t)L.env * C.N;
+    for (int o = 0; o < C.N; ++o)
+        obstacle_force_adj(C, g.obs, eN, o, in.px, in.py, in.vx, in.vy, L.pr.radius, L.dd, gFx, gFy,
+                           gi);
+    if (C.soft_walls)
+        wall_force_adj(C, in.px, in.py, in.vx, in.vy, L.pr.radius, L.dd, gFx, gFy, gi);
 }
 
 // Reverse of one agent's forces of a substep (published state and force adjoints /
@@ -779,17 +843,11 @@ __device__ __forceinline__ void wide_agent_adj(const Cst<T> &C, const Args<T> &g
             return;
         }
     }
-    if (C.N > 0) {
-        const size_t eN = (size_t)L.env * C.N;
-        for (int o = 0; o < C.N; ++o)
-            obstacle_force_adj(C, g.obs, eN, o, in.px, in.py, in.vx, in.vy, L.pr.radius, L.dd,
-                               gFx, gFy, gi);
-    }
-    if (C.soft_walls)
-        wall_force_adj(C, in.px, in.py, in.vx, in.vy, L.pr.radius, L.dd, gFx, gFy, gi);
+    wide_static_adj(C, g, L, in, gFx, gFy, gi);
 }
 
-template <typename T, bool DRONE, bool GRID, bool BOXES, int APT, unsigned F>
+// The backward rollout of box worlds.
+template <typename T, bool GRID, int APT, unsigned F>
 __global__ __launch_bounds__(1024) void k_wide_bwd(const Cst<T> Cin, const Args<T> g)
 {
     const Cst<T> C = fold_cst<F>(Cin);
@@ -800,7 +858,7 @@ __global__ __launch_bounds__(1024) void k_wide_bwd(const Cst<T> Cin, const Args<
     const WBoxLds<T> B = wide_box_lds<T>(smem, AP, wide_cells(C));
     const GridFrame<T> G = grid_frame(C, (const T *)nullptr);
     WLane<T> L[APT];
-    wide_lanes<T, BOXES, APT, F>(C, g, W, B, L);
+    wide_lanes<T, true, APT, F>(C, g, W, B, L);
     const size_t EA = (size_t)C.E * C.A;
     St<T> gs[APT];
 #pragma unroll
@@ -812,14 +870,14 @@ __global__ __launch_bounds__(1024) void k_wide_bwd(const Cst<T> Cin, const Args<
         for (int k = 0; k < APT; ++k) {
             if (L[k].active) {
                 if (t == g.nsteps - 1)
-                    add_adj<T, DRONE>(g.afin.f, L[k].idx, gs[k]);
+                    add_adj<T, false>(g.afin.f, L[k].idx, gs[k]);
                 else
-                    add_adj<T, DRONE>(g.atraj.f, (size_t)t * EA + L[k].idx, gs[k]);
+                    add_adj<T, false>(g.atraj.f, (size_t)t * EA + L[k].idx, gs[k]);
             }
             if (t == 0)
-                load_state<T, DRONE>(g.s0.f, L[k].idx, 0, st0[k]);
+                load_state<T, false>(g.s0.f, L[k].idx, 0, st0[k]);
             else
-                load_state<T, DRONE>(g.traj.f, L[k].idx, (size_t)(t - 1) * EA, st0[k]);
+                load_state<T, false>(g.traj.f, L[k].idx, (size_t)(t - 1) * EA, st0[k]);
             load_act(g.act, (size_t)t * EA + L[k].idx, C.ad, a[k]);
             for (int q = 0; q < 4; ++q) ga[k][q] = T(0);
         }
@@ -829,7 +887,7 @@ __global__ __launch_bounds__(1024) void k_wide_bwd(const Cst<T> Cin, const Args<
 #pragma unroll
             for (int k = 0; k < APT; ++k) in[k] = st0[k];
             for (int q = 0; q < s; ++q)
-                wide_substep<T, DRONE, GRID, BOXES, APT>(C, g, W, B, G, L, a, in, wsum);
+                wide_substep<T, false, GRID, true, APT>(C, g, W, B, G, L, a, in, wsum);
             T Fx[APT], Fy[APT];
             int32_t cut[APT];
 #pragma unroll
@@ -841,20 +899,20 @@ __global__ __launch_bounds__(1024) void k_wide_bwd(const Cst<T> Cin, const Args<
                 if (C.collisions) {
                     __syncthreads();
 #pragma unroll
-                    for (int k = 0; k < APT; ++k) wide_put(W, L[k], in[k], BOXES ? &B : nullptr);
+                    for (int k = 0; k < APT; ++k) wide_put(W, L[k], in[k], &B);
                     __syncthreads();
                     if (GRID) grid_build(W, C.A, G, wsum);
                 }
 #pragma unroll
                 for (int k = 0; k < APT; ++k)
-                    wide_agent_forces<T, GRID, BOXES>(C, g, W, B, G, L[k], in[k], Fx[k], Fy[k],
+                    wide_agent_forces<T, GRID, true>(C, g, W, B, G, L[k], in[k], Fx[k], Fy[k],
                                                       cut[k], nullptr);
             }
             St<T> gi[APT];
             T gFx[APT], gFy[APT];
 #pragma unroll
             for (int k = 0; k < APT; ++k)
-                integrate_adj<T, DRONE>(C, L[k].pr, in[k], a[k], Fx[k], Fy[k], gs[k], gi[k], ga[k],
+                integrate_adj<T, false>(C, L[k].pr, in[k], a[k], Fx[k], Fy[k], gs[k], gi[k], ga[k],
                                         gFx[k], gFy[k]);
             if (C.needs_forces) {
                 if (C.collisions) {
@@ -869,7 +927,7 @@ __global__ __launch_bounds__(1024) void k_wide_bwd(const Cst<T> Cin, const Args<
                 }
 #pragma unroll
                 for (int k = 0; k < APT; ++k)
-                    wide_agent_adj<T, GRID, BOXES>(C, g, W, B, G, L[k], in[k], gFx[k], gFy[k],
+                    wide_agent_adj<T, GRID, true>(C, g, W, B, G, L[k], in[k], gFx[k], gFy[k],
                                                    cut[k], gi[k]);
             }
 #pragma unroll
@@ -884,7 +942,7 @@ __global__ __launch_bounds__(1024) void k_wide_bwd(const Cst<T> Cin, const Args<
     }
 #pragma unroll
     for (int k = 0; k < APT; ++k)
-        if (L[k].active) store_adj<T, DRONE>(g.a0.f, L[k].idx, gs[k]);
+        if (L[k].active) store_adj<T, false>(g.a0.f, L[k].idx, gs[k]);
 }
 
 // ---------------------------------------------------------------------- launchers
@@ -892,7 +950,7 @@ __global__ __launch_bounds__(1024) void k_wide_bwd(const Cst<T> Cin, const Args<
 // Threads of the movable-body kernels' workgroup (one per agent slot, at most 1024 agents).
 template <typename T> inline int wide_threads(int A) { return ((A + 63) / 64) * 64; }
 
-template <typename T> size_t wide_shm(const Cst<T> &C, bool boxes = false)
+template <typename T> size_t wide_shm(const Cst<T> &C, bool boxes)
 {
     const int AP = wide_geom(C.A).slots, NC = C.grid_bins > 0 ? C.grid_bins * C.grid_bins : 0;
     return boxes ? wide_box_lds_bytes<T>(AP, NC) : wide_lds_bytes<T>(AP, NC);
@@ -903,7 +961,7 @@ void launch_wide_lists(const Cst<T> &C, const T *pos, const T *frame, int32_t *i
                        int32_t *tru, hipStream_t st)
 {
     const dim3 grid(C.E), block(wide_geom(C.A).threads);
-    const size_t shm = wide_shm<T>(C);
+    const size_t shm = wide_shm<T>(C, false);
     if (C.grid_bins > 0)
         hipLaunchKernelGGL((k_wide_lists<T, true>), grid, block, shm, st, C, pos, frame, idx, cnt, tru);
     else
@@ -929,62 +987,6 @@ void launch_grid_frame(const T *pos, int64_t n, T radius, int bins, void *scratc
                        FRAME_BLOCK, part, radius, bins, frame);
     hipLaunchKernelGGL((k_grid_frame<T>), dim3(1), dim3(256), 0, st, (const T *)part, nb, radius,
                        bins, frame);
-}
-
-// boxes: a box world (box agents or wheel contacts; never with drones).
-#define SWARP_WIDE_DISPATCH_APT(KERNEL, APT)                                                           \
-    if (drone) {                                                                                       \
-        if (grid) hipLaunchKernelGGL((KERNEL<T, true, true, false, APT, FT_ALL>), g, b, shm, st, C, a);  \
-        else hipLaunchKernelGGL((KERNEL<T, true, false, false, APT, FT_ALL>), g, b, shm, st, C, a);      \
-    } else if (boxes) {                                                                                \
-        if (grid) hipLaunchKernelGGL((KERNEL<T, false, true, true, APT, FT_ALL>), g, b, shm, st, C, a);  \
-        else hipLaunchKernelGGL((KERNEL<T, false, false, true, APT, FT_ALL>), g, b, shm, st, C, a);      \
-    } else {                                                                                           \
-        if (grid) hipLaunchKernelGGL((KERNEL<T, false, true, false, APT, FT_ALL>), g, b, shm, st, C, a); \
-        else hipLaunchKernelGGL((KERNEL<T, false, false, false, APT, FT_ALL>), g, b, shm, st, C, a);     \
-    }
-// The launchers of one agents-per-thread count (each count its own compilation unit).
-template <typename T, int APT>
-void launch_wide_fwd_apt(bool drone, bool boxes, const Cst<T> &C, const Args<T> &a,
-                         hipStream_t st)
-{
-    const dim3 g(C.E), b(wide_geom(C.A).threads);
-    const size_t shm = wide_shm<T>(C, boxes);
-    const bool grid = C.grid_bins > 0;
-    SWARP_WIDE_DISPATCH_APT(k_wide_fwd, APT)
-}
-
-template <typename T, int APT>
-void launch_wide_bwd_apt(bool drone, bool boxes, const Cst<T> &C, const Args<T> &a,
-                         hipStream_t st)
-{
-    const dim3 g(C.E), b(wide_geom(C.A).threads);
-    const size_t shm = wide_shm<T>(C, boxes);
-    const bool grid = C.grid_bins > 0;
-    SWARP_WIDE_DISPATCH_APT(k_wide_bwd, APT)
-}
-#undef SWARP_WIDE_DISPATCH_APT
-
-template <typename T>
-inline void launch_wide_fwd(bool drone, bool boxes, const Cst<T> &C, const Args<T> &a,
-                            hipStream_t st)
-{
-    switch (wide_geom(C.A).apt) {
-    case 1: launch_wide_fwd_apt<T, 1>(drone, boxes, C, a, st); break;
-    case 2: launch_wide_fwd_apt<T, 2>(drone, boxes, C, a, st); break;
-    default: launch_wide_fwd_apt<T, 4>(drone, boxes, C, a, st); break;
-    }
-}
-
-template <typename T>
-inline void launch_wide_bwd(bool drone, bool boxes, const Cst<T> &C, const Args<T> &a,
-                            hipStream_t st)
-{
-    switch (wide_geom(C.A).apt) {
-    case 1: launch_wide_bwd_apt<T, 1>(drone, boxes, C, a, st); break;
-    case 2: launch_wide_bwd_apt<T, 2>(drone, boxes, C, a, st); break;
-    default: launch_wide_bwd_apt<T, 4>(drone, boxes, C, a, st); break;
-    }
 }
 
 }  // namespace swarp

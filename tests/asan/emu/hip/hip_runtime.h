@@ -221,6 +221,7 @@ inline long long min(long long a, long long b) { return a < b ? a : b; }
 inline long long max(long long a, long long b) { return a > b ? a : b; }
 
 inline int atomicAdd(int *p, int v) { return __atomic_fetch_add(p, v, __ATOMIC_SEQ_CST); }
+inline int atomicExch(int *p, int v) { return __atomic_exchange_n(p, v, __ATOMIC_SEQ_CST); }
 
 inline float __builtin_amdgcn_sqrtf(float x) { return sqrtf(x); }
 inline double __builtin_amdgcn_rcp(double x) { return 1.0 / x; }

@@ -6,8 +6,10 @@ import numpy as np
 import pytest
 import torch
 
-from oracle.oracle import Oracle
+from hip_helpers import hip_run, make_stepper, oracle_run, rel
+from oracle.oracle import Oracle, pack_state
 from swarp_amd import NeighborGrid
+from swarp_amd.config import AgentConfig, DynamicsModel, WorldConfig
 
 pytestmark = pytest.mark.gpu
 
@@ -57,3 +59,69 @@ def test_grid_lists_in_crowded_cells(A, spread):
     assert np.array_equal(g.neighbor_idx.cpu().numpy(), oi)
     assert np.array_equal(g.neighbor_count.cpu().numpy(), oc)
     assert np.array_equal(g.neighbor_true_count.cpu().numpy(), ot)
+
+
+@pytest.mark.parametrize("E,A,T,S,half,kw", [
+    (5, 65, 6, 4, 2.2, {}),                               # just past a wavefront, sparse
+    (3, 256, 5, 3, 4.0, {}),                              # every slot of the small hash in use
+    (2, 200, 4, 4, 0.9, {}),                              # candidate lists overflow: full traversal
+    (3, 130, 5, 2, 1.6, dict(max_neighbors=3)),           # lists truncated among few candidates
+    (2, 90, 5, 2, 0.8, dict(neighbor_radius=0.3, max_neighbors=5)),
+    (2, 128, 6, 1, 1.5, {}),                              # one substep: no skin
+    (2, 600, 4, 2, 5.0, {}),                              # uniform grid, sparse
+    (2, 600, 4, 3, 1.7, dict(max_neighbors=4)),           # uniform grid, truncated and overflowing
+    (2, 70, 6, 3, 1.5, dict(neighbor_method="uniform_grid", uniform_bins=5)),
+    (2, 1030, 3, 2, 7.0, {}),                             # two agents per thread
+    (1, 1500, 3, 2, 8.0, dict(neighbor_method="brute")),
+    (1, 2060, 2, 2, 9.0, {}),                             # four agents per thread
+    (1, 3584, 2, 2, 12.0, dict(neighbor_method="brute")),  # the largest env: the shortest lists
+    (2, 100, 4, 2, 1.6, dict(f64=True)),
+    (1, 2048, 2, 2, 10.0, dict(f64=True, neighbor_method="brute")),
+    (3, 80, 5, 4, 1.5, dict(shift=40000.0)),              # beyond the hash's certain range
+    (3, 96, 5, 4, 2.0, dict(fast=6.0)),                   # agents outrun the skin
+    (3, 96, 5, 2, 1.1, dict(mixed=True)),                 # diff-drive and bicycle
+])
+def test_swarm_rollout(E, A, T, S, half, kw):
+    """States bit-exact with the oracle (float64: 1e-12), gradients within the bars; with and
+    without the tape the same bits."""
+    kw = dict(kw)
+    dt = np.float64 if kw.pop("f64", False) else np.float32
+    shift, fast, mixed = kw.pop("shift", 0.0), kw.pop("fast", 0.0), kw.pop("mixed", False)
+    rng = np.random.default_rng(A + S)
+    cfgs = [AgentConfig(radius=0.05) for _ in range(A)]
+    if mixed:
+        cfgs = [AgentConfig(model=DynamicsModel.DIFF_DRIVE if k % 2 else
+                            DynamicsModel.KINEMATIC_BICYCLE, radius=0.05) for k in range(A)]
+    ad, nf = 2, 5
+    s0 = {"pos": rng.uniform(-half, half, size=(E, A, 2)) + shift,
+          "theta": rng.uniform(-np.pi, np.pi, size=(E, A))}
+    acts = rng.uniform(-1, 1, size=(T, E, A, 2))
+    bounds = (shift - half, shift + half, shift - half, shift + half)
+    if fast:  # drones keep their initial velocity, whatever max_speed says
+        cfgs = [AgentConfig(model=DynamicsModel.DRONE, radius=0.1) for _ in range(A)]
+        ad, nf, bounds = 4, 9, None
+        s0["vel"] = rng.uniform(-fast, fast, size=(E, A, 2))
+        s0["attitude"] = np.broadcast_to([0.0, 0.0, 0.0, 1.0], (E, A, 4))
+        acts = rng.uniform(0, 10, size=(T, E, A, 4))
+    s0, acts = pack_state(s0).astype(dt), acts.astype(dt)
+    world = WorldConfig(collision_k=100.0, collision_c=1.0, collision_margin=0.025, bounds=bounds,
+                        **kw)
+    w = rng.normal(size=(T, E, A, 16)) * (0.01 if fast else 1.0)
+    if nf == 5:
+        w[..., 7:] = 0.0
+    td = torch.float32 if dt == np.float32 else torch.float64
+    on = make_stepper(cfgs, world, 0.05, S, td)
+    off = make_stepper(cfgs, world, 0.05, S, td)
+    off.use_tape = False
+    assert on.wide and on.tape_bytes(E, ad, T) > 0 and off.tape_bytes(E, ad, T) == 0
+    a, b = hip_run(on, s0, acts, w, dt), hip_run(off, s0, acts, w, dt)
+    for x, y in zip(a, b):
+        assert np.array_equal(x, y), "the tape changes a result"
+    o = oracle_run(cfgs, world, 0.05, S, s0, acts, w, dt)
+    cols = slice(0, 16 if fast else 7)
+    if dt == np.float32:
+        assert np.array_equal(a[0][..., cols], o[0][..., cols])
+    else:
+        assert rel(a[0][..., cols], o[0][..., cols]) <= 1e-12
+    tol = 1e-5 if dt == np.float32 else 1e-12  # the gradient bars of test_hip_wide.py
+    assert rel(a[2], o[2]) <= tol and rel(a[1][..., cols], o[1][..., cols]) <= tol
