@@ -13,6 +13,9 @@
 //     env slot hold NaN positions, which fail every membership test, so the LDS reads of
 //     a scan are issued back to back and waited on once;
 //   * the next step's inputs are loaded one step ahead.
+// Parameter rows are per agent or per env and agent (each lane reads its own once, so a
+// randomized fleet runs here too): 3000 envs x 16 agents, 16 steps of 4 substeps with per-env
+// rows take 83 / 64 us forward / backward, on the generic kernels 117 / 181.
 #pragma once
 #include "common.hpp"
 
@@ -304,7 +307,7 @@ __global__ __launch_bounds__(64) void k_holo_fwd(const Cst<T> C, const Args<T> g
     const bool real = me < C.A;
     const bool active = real && env < C.E;
     const size_t i = (size_t)(env < C.E ? env : 0) * C.A + (real ? me : 0);
-    const T *prow = g.params + (real ? me : 0) * 22;
+    const T *prow = g.params + (C.per_env ? i : (size_t)(real ? me : 0)) * 22;
     const T ra = prow[0], mass = prow[1], vmax = prow[2];
     const T dt = C.sub_dt, dtm = dt / mass, dd = T(1) + C.c * C.sub_dt / mass;
     const Dv<T> ddv = divisor(dd, true);
@@ -412,7 +415,7 @@ __global__ __launch_bounds__(64) void k_holo_bwd(const Cst<T> C, const Args<T> g
     const bool real = me < C.A;
     const bool active = real && env < C.E;
     const size_t i = (size_t)(env < C.E ? env : 0) * C.A + (real ? me : 0);
-    const T *prow = g.params + (real ? me : 0) * 22;
+    const T *prow = g.params + (C.per_env ? i : (size_t)(real ? me : 0)) * 22;
     const T ra = prow[0], mass = prow[1], vmax = prow[2];
     const T dt = C.sub_dt, dtm = dt / mass, dd = T(1) + C.c * C.sub_dt / mass;
     const Dv<T> ddv = divisor(dd, true);

@@ -271,8 +271,7 @@ template <typename T> static int wide_lds_check(const swarp_desc_t *d, bool list
 static bool lean_ok(const swarp_desc_t *d)
 {
     return !wide_path(d) && d->holo_velocity_only && !d->has_drone && d->n_obstacles == 0 && !d->clamp_bounds &&
-           d->integrator == SWARP_EULER && !d->has_boxes && !d->wheel_contacts &&
-           !d->params_per_env;
+           d->integrator == SWARP_EULER && !d->has_boxes && !d->wheel_contacts;
 }
 
 // Byte offsets of the tape regions (see lean.hpp); total == 0: no tape.  The specialised
