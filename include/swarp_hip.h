@@ -262,13 +262,15 @@ int swarp_rollout_bwd_ob_check(const swarp_desc_t *desc);
 /* Body tape: per substep and movable body, the body pass's result -- the body's new pose
  * and velocity, the new angle's cos / sin, its contact force and torque -- written by the
  * forward so that the backward's recompute of each step reads it instead of evaluating
- * the pass again (the agents' forces are still recomputed from the checkpoints).  Bodies
- * are counted in root order (the obstacle indices o with body[o] = o and kind[o] = 1);
+ * the pass again; and, up to 64 agents per env with index-ordered lists, behind those
+ * records what the agents felt (forces and touching agents of the few that feel any, the
+ * shapes touched), read instead of evaluating their forces again.  Bodies are counted in root order (the obstacle indices o with body[o] = o and kind[o] = 1);
  * a tape may hold the first n_bodies of them, and the backward evaluates the others.
  * No counterpart in the reference: its body pass runs on untaped steps and is not
  * differentiated (swarp/core/stepper.py:952-991).
  * Writes in *bytes the size of the tape of a T-step rollout holding n_bodies bodies
- * (1 <= n_bodies <= n_obstacles): T * substeps * n_envs * n_bodies * 12 scalars. */
+ * (1 <= n_bodies <= n_obstacles).  A tape of T * substeps * n_envs * n_bodies * 12 scalars
+ * holds the body records alone and is taken too (a slower backward, the same results). */
 int swarp_ob_tape_bytes(const swarp_desc_t *desc, int32_t T, int32_t n_bodies, uint64_t *bytes);
 
 /* swarp_rollout_fwd_ob that also writes the body tape (device memory owned by the caller;

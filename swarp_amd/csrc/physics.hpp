@@ -707,12 +707,12 @@ __device__ __forceinline__ bool box_force_cs(const Cst<T> &C, T px, T py, T vx, 
 }
 
 template <typename T, typename DD>
-__device__ __forceinline__ void box_force(const Cst<T> &C, T px, T py, T vx, T vy, T cx0, T cy0,
+__device__ __forceinline__ bool box_force(const Cst<T> &C, T px, T py, T vx, T vy, T cx0, T cy0,
                                           T ang, T hx, T hy, T reach, const DD &dd, T vox, T voy,
                                           T om, T &fx, T &fy)
 {
-    box_force_cs(C, px, py, vx, vy, cx0, cy0, m_cos(ang), m_sin(ang), hx, hy, reach, dd, vox,
-                 voy, om, fx, fy);
+    return box_force_cs(C, px, py, vx, vy, cx0, cy0, m_cos(ang), m_sin(ang), hx, hy, reach, dd,
+                        vox, voy, om, fx, fy);
 }
 
 template <typename T>

@@ -573,13 +573,49 @@ template <typename T> static int fill_obtab(const swarp_desc_t *d, ObTab<T> &tb)
     return 0;
 }
 
-// Bodies a body tape of `bytes` holds for a T-step rollout of d (0: not a whole number of
-// per-body slices, or none).
-template <typename T> static int64_t ob_tape_roots(const swarp_desc_t *d, int32_t nT, uint64_t bytes)
+// The body tape of a T-step rollout with n_bodies records per substep and env, and behind it
+// the lane tape (narrow envs; up to LANE_TAPE_MAX, beyond which the backward evaluates the
+// forces again).
+struct ObTapeLayout {
+    uint64_t lane, total;  // lane == 0: no lane tape
+};
+constexpr uint64_t LANE_TAPE_MAX = 16ull << 30;
+
+template <typename T>
+static ObTapeLayout ob_tape_layout(const swarp_desc_t *d, int32_t nT, int32_t n_bodies)
 {
+    ObTapeLayout L = {0, (uint64_t)nT * d->substeps * d->n_envs * n_bodies * BODY_REC * sizeof(T)};
+    if (wide_path(d)) return L;
+    const int PA = body_pa<T>(d);
+    const uint64_t waves = (d->n_envs + 64 / PA - 1) / (64 / PA);
+    const uint64_t lanes = (uint64_t)nT * d->substeps * waves * lane_tape_rec(PA, sizeof(T));
+    if (lanes > LANE_TAPE_MAX) return L;
+    L.lane = align256(L.total);
+    L.total = L.lane + lanes;
+    return L;
+}
+
+// The tape pointers of a rollout from a tape of `bytes`: as many bodies as the layout of that
+// size holds, or the body records alone (T * substeps * n_envs * 12 scalars per body).
+template <typename T>
+static int ob_tape_ptrs(const swarp_desc_t *d, int32_t nT, void *tape, uint64_t bytes, ObIO<T> &io)
+{
+    if (!tape) return 0;
+    for (int32_t r = 1; r <= d->n_obstacles; ++r) {
+        const ObTapeLayout L = ob_tape_layout<T>(d, nT, r);
+        if (L.total != bytes) continue;
+        io.tape = (T *)tape;
+        io.tape_roots = r;
+        if (L.lane && ((uintptr_t)tape & 7) == 0) io.ltape = (unsigned char *)tape + L.lane;
+        return 0;
+    }
     const uint64_t per = (uint64_t)nT * d->substeps * d->n_envs * BODY_REC * sizeof(T);
-    if (per == 0 || bytes % per != 0) return 0;
-    return (int64_t)(bytes / per);
+    if (bytes >= per && bytes % per == 0 && bytes / per <= (uint64_t)d->n_obstacles) {
+        io.tape = (T *)tape;
+        io.tape_roots = (int)(bytes / per);
+        return 0;
+    }
+    return fail("tape_bytes is not swarp_ob_tape_bytes of 1..n_obstacles bodies");
 }
 
 template <typename T>
@@ -604,14 +640,8 @@ static int rollout_fwd_ob(const swarp_desc_t *d, int32_t nT, const swarp_state_t
     if (nT > 1) copy_fields<T>(traj, a.traj.f);
     a.act = (const T *)act;
     a.nsteps = nT;
-    ObIO<T> io = {(const T *)ob0, (T *)ob_traj, nullptr, nullptr, nullptr, 0};
-    if (tape) {
-        const int64_t r = ob_tape_roots<T>(d, nT, tape_bytes);
-        if (r < 1 || r > d->n_obstacles)
-            return fail("tape_bytes is not swarp_ob_tape_bytes of 1..n_obstacles bodies");
-        io.tape = (T *)tape;
-        io.tape_roots = (int)r;
-    }
+    ObIO<T> io = {(const T *)ob0, (T *)ob_traj, nullptr, nullptr, nullptr, 0, nullptr};
+    if (ob_tape_ptrs<T>(d, nT, tape, tape_bytes, io)) return -1;
     if (wide_path(d)) {
         // the wide kernels keep no body tape (their backward evaluates the pass again)
         io.tape = nullptr;
@@ -652,14 +682,8 @@ static int rollout_bwd_ob(const swarp_desc_t *d, int32_t nT, const swarp_state_t
     a.act = (const T *)act;
     a.aact = (T *)aact;
     a.nsteps = nT;
-    ObIO<T> io = {(const T *)ob0, (T *)ob_traj, (const T *)aob_traj, (T *)aob0, nullptr, 0};
-    if (tape) {
-        const int64_t r = ob_tape_roots<T>(d, nT, tape_bytes);
-        if (r < 1 || r > d->n_obstacles)
-            return fail("tape_bytes is not swarp_ob_tape_bytes of 1..n_obstacles bodies");
-        io.tape = (T *)tape;
-        io.tape_roots = (int)r;
-    }
+    ObIO<T> io = {(const T *)ob0, (T *)ob_traj, (const T *)aob_traj, (T *)aob0, nullptr, 0, nullptr};
+    if (ob_tape_ptrs<T>(d, nT, (void *)tape, tape_bytes, io)) return -1;
     if (wide_path(d)) {
         if (wbody_lds_check<T>(d, true)) return -1;
         io.tape = nullptr;
@@ -802,8 +826,8 @@ int swarp_ob_tape_bytes(const swarp_desc_t *desc, int32_t T, int32_t n_bodies, u
     if (T < 1) return fail("T must be >= 1");
     if (n_bodies < 1 || n_bodies > desc->n_obstacles)
         return fail("n_bodies must lie in [1, n_obstacles]");
-    const uint64_t ts = desc->dtype == SWARP_F32 ? 4 : 8;
-    *bytes = (uint64_t)T * desc->substeps * desc->n_envs * n_bodies * BODY_REC * ts;
+    *bytes = desc->dtype == SWARP_F32 ? ob_tape_layout<float>(desc, T, n_bodies).total
+                                      : ob_tape_layout<double>(desc, T, n_bodies).total;
     return 0;
 }
 
