@@ -338,6 +338,87 @@ template <typename M> __device__ __forceinline__ M cap_list(M incl, int K)
     return incl ^ rest;
 }
 
+// Padded list rows leave a wave straight from the lists' masks.  A row of K 4-byte slots written
+// to LDS by its lane, slot by slot, puts every lane's k-th word in one bank when K is a
+// multiple of 32 and a few otherwise, and holds 256 K bytes of LDS; instead each row's mask and
+// its first four members (a byte each: most rows hold no more) go to LDS, and the wave's lanes
+// form the output 16 bytes at a time in memory order.
+//   row_put   one lane's row r
+//   rows_out  `n` consecutive rows from row r0 to dst
+template <typename M> struct RowLds {
+    M mask[64];
+    uint32_t four[64];
+};
+
+template <typename M> __device__ __forceinline__ void row_put(RowLds<M> &R, int r, M m)
+{
+    R.mask[r] = m;
+    uint32_t w = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        if (m) w |= (uint32_t)m_ctz(m) << (8 * k);
+        m &= m - 1;
+    }
+    R.four[r] = w;
+}
+
+template <typename M> __device__ __forceinline__ int32_t row_slot(const RowLds<M> &R, int r, int k)
+{
+    if (k < 4) return (int32_t)((R.four[r] >> (8 * k)) & 0xffu);
+    M m = R.mask[r];
+    if (k >= m_popc(m)) return 0;
+    for (int q = 0; q < k; ++q) m &= m - 1;
+    return m_ctz(m);
+}
+
+template <typename M>
+__device__ __forceinline__ void rows_out(int32_t *dst, const RowLds<M> &R, int r0, int n, int K,
+                                         int lane)
+{
+    const int per = (K & 3) == 0 && ((uintptr_t)dst & 15u) == 0u ? 4 : 1;  // slots per store
+    const int P = K / per, total = n * P;  // stores per row, and in all
+    int r = r0 + lane / P, c = lane % P;
+    const int dr = 64 / P, dc = 64 % P;
+    if (per == 4) {
+        for (int q = lane; q < total; q += 64) {
+            int4 v = make_int4(0, 0, 0, 0);
+            if (c == 0) {
+                const uint32_t w = R.four[r];
+                v = make_int4(w & 0xffu, (w >> 8) & 0xffu, (w >> 16) & 0xffu, w >> 24);
+            } else {
+                M m = R.mask[r];
+                if (4 * c < m_popc(m)) {
+                    for (int k = 0; k < 4 * c; ++k) m &= m - 1;
+                    int e[4];
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        e[k] = m ? m_ctz(m) : 0;
+                        m &= m - 1;
+                    }
+                    v = make_int4(e[0], e[1], e[2], e[3]);
+                }
+            }
+            ((int4 *)dst)[q] = v;
+            r += dr;
+            c += dc;
+            if (c >= P) {
+                c -= P;
+                ++r;
+            }
+        }
+        return;
+    }
+    for (int q = lane; q < total; q += 64) {
+        dst[q] = row_slot(R, r, c);
+        r += dr;
+        c += dc;
+        if (c >= P) {
+            c -= P;
+            ++r;
+        }
+    }
+}
+
 // ------------------------------------------------------------- feature profiles
 //
 // The generic and body kernels are instantiated per feature profile F: a bit set of the

@@ -11,7 +11,10 @@
 // Layout: one lane per (env, agent) as in the step kernels -- an env is PA consecutive
 // lanes of a wave64, so the env's lists and its reward reduction stay inside the wave
 // (positions and per-agent terms in LDS, no global atomics).  Observation rows are
-// assembled in LDS and leave as contiguous, coalesced stores when they fit.
+// assembled in LDS and leave as contiguous, coalesced stores when they fit; list rows leave
+// from their masks (rows_out).  Writing bounds the pass (319 MB at 16000 envs x 64 agents, of
+// which 131 MB are list slots); with the list rows staged in LDS as well, their bank conflicts
+// and the 15 KB a wave held did: 102 -> 51 us.
 // Instantiated by k_nav.hip.
 #pragma once
 #include "common.hpp"
@@ -53,16 +56,17 @@ __global__ __launch_bounds__(64) void k_nav(const Cst<T> C, const NavArgs<T> g)
     typedef typename MaskT<PA>::type M;
     __shared__ T lx[64], ly[64], lvx[64], lvy[64], lra[64], lsh[64];
     __shared__ int log_[64];
+    __shared__ RowLds<M> rows;
     extern __shared__ __align__(16) unsigned char nav_dyn[];
-    // staged output rows: observation rows [64][W], then list rows [64][K]
+    // staged observation rows [EPW * A][W]
     T *row_lds = reinterpret_cast<T *>(nav_dyn);
-    int32_t *idx_lds = reinterpret_cast<int32_t *>(nav_dyn + (size_t)64 * g.W * sizeof(T));
 
     const int lane = threadIdx.x, agent = lane % PA, base = lane - agent;
     const int env = blockIdx.x * (64 / PA) + lane / PA;
     const bool real = agent < C.A;
     const bool active = real && env < C.E;
     const size_t i = active ? (size_t)env * C.A + agent : 0;
+    const int row = (lane / PA) * C.A + agent;  // of the wave's output rows (real agents)
     const bool reset_hit = active && g.rmask != nullptr && g.rmask[env] != 0;
     // an obs-only pass (auto-reset) recomputes only the envs it resets: the others'
     // positions are unchanged since the step pass that already wrote every output
@@ -94,18 +98,7 @@ __global__ __launch_bounds__(64) void k_nav(const Cst<T> C, const NavArgs<T> g)
     const M incl = scan_all<T, PA>(lx, ly, base, C.A, agent, px, py, C.t_nbr, C.t_nbr, cd);
     const M m = cap_list(incl, C.K);
     const int n = m_popc(m);
-    if (g.stage || work) {
-        int32_t *irow = g.stage ? idx_lds + (size_t)lane * C.K : g.idx + i * C.K;
-        M mm = m;
-        for (int k = 0; k < C.K; ++k) {
-            int v = 0;
-            if (k < n) {
-                v = m_ctz(mm);
-                mm &= mm - 1;
-            }
-            irow[k] = v;
-        }
-    }
+    if (real) row_put(rows, row, m);
     if (work) {
         g.cnt[i] = n;
         if (g.tru) g.tru[i] = m_popc(incl);
@@ -139,8 +132,8 @@ __global__ __launch_bounds__(64) void k_nav(const Cst<T> C, const NavArgs<T> g)
     // observation row (_obs_row, :41-89)
     const int W = g.W, KO = g.k_obs;
     {
-        T *dst = g.stage ? row_lds + (size_t)lane * W : g.obs + i * W;
-        const bool put = g.stage || work;
+        T *dst = g.stage ? row_lds + (size_t)row * W : g.obs + i * W;
+        const bool put = g.stage ? real : work;
         if (put) {
             dst[0] = px;
             dst[1] = py;
@@ -195,24 +188,18 @@ __global__ __launch_bounds__(64) void k_nav(const Cst<T> C, const NavArgs<T> g)
         }
     }
 
-    if (g.stage) {
-        // an env's rows are A consecutive rows both in LDS (lanes e*PA .. e*PA+A-1) and in
-        // memory, so each env leaves as one contiguous block; with no pad slots (A == PA)
-        // and every env written, the whole wave's rows are one block
+    {
+        // an env's rows are A consecutive rows in LDS and in memory, and so are the wave's envs':
+        // a full pass writes them all as one block, an obs-only pass those of the reset envs
         __syncthreads();
         const int env0 = blockIdx.x * (64 / PA);
         const int n_env = min(64 / PA, C.E - env0);
-        if (g.full_pass != 0 && PA == C.A) {
-            const size_t first = (size_t)env0 * C.A;
-            wave_copy(g.obs + first * W, row_lds, n_env * C.A * W, lane);
-            wave_copy(g.idx + first * C.K, idx_lds, n_env * C.A * C.K, lane);
-        } else {
-            for (int e = 0; e < n_env; ++e) {
-                if (g.full_pass == 0 && !(g.rmask != nullptr && g.rmask[env0 + e] != 0)) continue;
-                const size_t first = (size_t)(env0 + e) * C.A;
-                wave_copy(g.obs + first * W, row_lds + (size_t)e * PA * W, C.A * W, lane);
-                wave_copy(g.idx + first * C.K, idx_lds + (size_t)e * PA * C.K, C.A * C.K, lane);
-            }
+        const int blocks = g.full_pass != 0 ? 1 : n_env, per = g.full_pass != 0 ? n_env * C.A : C.A;
+        for (int e = 0; e < blocks; ++e) {
+            if (g.full_pass == 0 && !(g.rmask != nullptr && g.rmask[env0 + e] != 0)) continue;
+            const size_t first = (size_t)env0 * C.A + (size_t)e * per;
+            if (g.stage) wave_copy(g.obs + first * W, row_lds + (size_t)e * per * W, per * W, lane);
+            rows_out(g.idx + first * C.K, rows, e * per, per, C.K, lane);
         }
     }
 
