@@ -159,7 +159,7 @@ __device__ inline void block_exclusive_scan(int32_t *v, int n, int32_t *wsum)
 // default bins) instead of a pass over all smaller indices: the counting atomics hand every
 // agent a slot of its cell in arrival order, the agent counts its cell's members of smaller
 // index there, and the second scatter puts the cell in index order.  The O(A) pass bound
-// the list build (200 envs x 1000 agents: 45 -> 30 us) and every kernel that sorts at each
+// the list build (200 envs x 1000 agents: 45 -> 30 us of it) and every kernel that sorts at each
 // substep (48 x 2000 agents, 8 steps of 2 substeps: forward 3.16 -> 0.52 ms).
 template <typename T>
 __device__ inline void grid_build(const WideLds<T> &W, int A, const GridFrame<T> &G,
@@ -220,20 +220,28 @@ __device__ __forceinline__ int visit_list(const WideLds<T> &W, int A, const Grid
         }
         return n;
     }
+    // a row of the block is one run of the sort, taken four agents at a time so that their
+    // reads are waited for together
     const int k = W.key[i], cx = k % G.bins, cy = k / G.bins;
+    const int x0 = cx > 0 ? cx - 1 : 0, x1 = cx + 1 < G.bins ? cx + 1 : G.bins - 1;
     for (int sy = 0; sy < 3; ++sy) {
         const int ny = cy + sy - 1;
         if (ny < 0 || ny >= G.bins) continue;
-        for (int sx = 0; sx < 3; ++sx) {
-            const int nx = cx + sx - 1;
-            if (nx < 0 || nx >= G.bins) continue;
-            const int c = ny * G.bins + nx, c0 = W.cstart[c], c1 = W.cstart[c + 1];
-            for (int si = c0; si < c1; ++si) {
-                const int j = W.sorted[si];
-                const T dx = W.px[j] - px, dy = W.py[j] - py;
-                const T d2 = dx * dx + dy * dy;
-                if (!(d2 <= t_nbr) || j == i) continue;
-                if (n < limit) f(j, (3 * sy + sx) * WIDE_MAX_AGENTS + (si - c0));
+        const int q1 = W.cstart[ny * G.bins + x1 + 1];
+        for (int q = W.cstart[ny * G.bins + x0]; q < q1; q += 4) {
+            int js[4];
+            unsigned hits = 0;
+#pragma unroll
+            for (int u = 0; u < 4; ++u) js[u] = q + u < q1 ? W.sorted[q + u] : i;
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const T dx = W.px[js[u]] - px, dy = W.py[js[u]] - py;
+                hits |= dx * dx + dy * dy <= t_nbr && js[u] != i ? 1u << u : 0u;
+            }
+            for (; hits; hits &= hits - 1) {
+                const int j = W.sorted[q + __builtin_ctz(hits)];
+                if (n < limit)
+                    f(j, (3 * sy + W.key[j] % G.bins - cx + 1) * WIDE_MAX_AGENTS + W.rank[j]);
                 ++n;
                 if (!count_all && n >= limit) return n;
             }
@@ -392,16 +400,27 @@ __host__ __device__ inline WideGeom wide_geom(int A)
     return {apt, th, th * apt};
 }
 
+// Where the staged rows of k_wide_lists begin, behind the agents' staging.
+template <typename T> __host__ __device__ inline size_t wide_lists_offset(int AP, int bins)
+{
+    return (wide_lds_bytes<T>(AP, bins * bins) + 15) / 16 * 16;
+}
+
 // Padded lists, counts and true counts of one env per workgroup (brute or grid order).
-template <typename T, bool GRID>
+// STAGE: the rows are collected in LDS, slot by slot with the agents side by side (16-bit ids,
+// after the staging), and leave in memory order, 4 or 16 bytes a lane; else (rows too long)
+// each thread writes its own, a store of 64 cache lines per slot.  200 envs x 1000 agents,
+// K = 16: 30 -> 16 us with the traversal's runs.
+template <typename T, bool GRID, bool STAGE>
 __global__ __launch_bounds__(1024) void k_wide_lists(const Cst<T> C, const T *pos, const T *frame,
                                                      int32_t *idx, int32_t *cnt, int32_t *tru)
 {
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ int32_t wsum[16];
-    const int nt = blockDim.x, A = C.A, env = blockIdx.x;
+    const int nt = blockDim.x, A = C.A, env = blockIdx.x, K = C.K;
     const int AP = nt * wide_geom(A).apt;
     const WideLds<T> W = wide_lds<T>(smem, AP);
+    uint16_t *const slots = (uint16_t *)(smem + wide_lists_offset<T>(AP, GRID ? C.grid_bins : 0));
     const GridFrame<T> G = grid_frame(C, frame);
     for (int i = threadIdx.x; i < AP; i += nt) {
         const size_t row = (size_t)env * A + (i < A ? i : 0);
@@ -412,13 +431,40 @@ __global__ __launch_bounds__(1024) void k_wide_lists(const Cst<T> C, const T *po
     if (GRID) grid_build(W, A, G, wsum);
     for (int i = threadIdx.x; i < A; i += nt) {
         const size_t row = (size_t)env * A + i;
-        int32_t *out = idx + row * C.K;
-        const int n = visit_list<T, GRID>(W, A, G, i, W.px[i], W.py[i], C.t_nbr, C.K, true,
-                                          [&](int j, int32_t) { *out++ = j; });
-        const int c = n < C.K ? n : C.K;
-        for (int q = c; q < C.K; ++q) idx[row * C.K + q] = 0;
+        int32_t *out = idx + row * K;
+        int m = 0;
+        const int n = visit_list<T, GRID>(W, A, G, i, W.px[i], W.py[i], C.t_nbr, K, true,
+                                          [&](int j, int32_t) {
+                                              if (STAGE) slots[(m++) * AP + i] = (uint16_t)j;
+                                              else out[m++] = j;
+                                          });
+        const int c = n < K ? n : K;
+        if (STAGE) W.cut[i] = c;
+        else
+            for (int q = c; q < K; ++q) out[q] = 0;
         cnt[row] = c;
         if (tru) tru[row] = n;
+    }
+    if (!STAGE) return;
+    __syncthreads();
+    int32_t *dst = idx + (size_t)env * A * K;
+    const int per = (K & 3) == 0 && ((uintptr_t)dst & 15u) == 0u ? 4 : 1;  // slots per store
+    const int P = K / per, total = A * P;
+    int i = (int)threadIdx.x / P, k = (int)threadIdx.x % P * per;
+    const int di = nt / P, dk = nt % P * per;
+    for (int q = threadIdx.x; q < total; q += nt) {
+        const int c = W.cut[i];
+        int v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) v[u] = u < per && k + u < c ? slots[(k + u) * AP + i] : 0;
+        if (per == 4) ((int4 *)dst)[q] = make_int4(v[0], v[1], v[2], v[3]);
+        else dst[q] = v[0];
+        i += di;
+        k += dk;
+        if (k >= K) {
+            k -= K;
+            ++i;
+        }
     }
 }
 
@@ -961,11 +1007,18 @@ void launch_wide_lists(const Cst<T> &C, const T *pos, const T *frame, int32_t *i
                        int32_t *tru, hipStream_t st)
 {
     const dim3 grid(C.E), block(wide_geom(C.A).threads);
-    const size_t shm = wide_shm<T>(C, false);
-    if (C.grid_bins > 0)
-        hipLaunchKernelGGL((k_wide_lists<T, true>), grid, block, shm, st, C, pos, frame, idx, cnt, tru);
-    else
-        hipLaunchKernelGGL((k_wide_lists<T, false>), grid, block, shm, st, C, pos, frame, idx, cnt, tru);
+    const int AP = wide_geom(C.A).slots;
+    const size_t rows = wide_lists_offset<T>(AP, C.grid_bins) + (size_t)C.K * AP * sizeof(uint16_t);
+    const bool stage = rows + 16 * sizeof(int32_t) <= LDS_MAX;  // with the static wsum
+    const size_t shm = stage ? rows : wide_shm<T>(C, false);
+#define SWARP_LISTS(GRID)                                                                           \
+    {                                                                                               \
+        if (stage) hipLaunchKernelGGL((k_wide_lists<T, GRID, true>), grid, block, shm, st, C, pos, frame, idx, cnt, tru); \
+        else hipLaunchKernelGGL((k_wide_lists<T, GRID, false>), grid, block, shm, st, C, pos, frame, idx, cnt, tru); \
+    }
+    if (C.grid_bins > 0) SWARP_LISTS(true)
+    else SWARP_LISTS(false)
+#undef SWARP_LISTS
 }
 
 // `scratch`: device memory the two-launch reduction may overwrite (the list buffer the
