@@ -70,7 +70,7 @@ constexpr int BODY_REC = 12;
 // on a field that is not crowded), so only those lanes' entries are kept, packed in lane
 // order behind the masks that say whose they are:
 //   words  0 lanes with a force that is not +0, 1 lanes that touch an agent, 2 shapes that some
-//          lane touches (forces_b), 3 shapes that feel a reaction (body_sum), 4 whether some
+//          lane touches (forces_b), 3 shapes in contact with an agent (body_sum), 4 whether some
 //          list was truncated (then word 1's masks are not its reverse's, and the backward
 //          scans)
 //   FO     forces of the lanes of word 0, pairs
@@ -690,7 +690,9 @@ __device__ __forceinline__ void body_load(const ObTab<T> &tb, const T *od, const
 // the body (index order): the agents' reactions in agent order, then the contacts with
 // the shapes of other bodies and of the scenery in index order (swarp/core/bodies.py:
 // 423-501).  bm = SS.of(o).  `hit` (nullable; narrow envs, with `rec`): bit s % 64 set for each
-// shape s that feels a reaction in some env of the wave.
+// shape s that some agent of the wave's envs is in contact with.  That is the contact's own
+// branch and not a force other than zero: an agent at the very centre of a round shape exerts
+// none, but its derivative is the largest there is.
 template <typename T, typename X, bool SM>
 __device__ __forceinline__ void body_sum(const Cst<T> &C, const ObTab<T> &tb,
                                          const ShapeSets<T, SM> &SS, const X &L,
@@ -712,15 +714,17 @@ __device__ __forceinline__ void body_sum(const Cst<T> &C, const ObTab<T> &tb,
         const T bound = shape_bound(ty, ro, hx, hy);
         // the agents' reactions, in agent order
         T f0 = T(0), f1 = T(0), tq = T(0);
+        bool felt = false;
         if (L.active() && !b_apart(st.px - csx, st.py - csy, br.r + bound + C.margin)) {
             T r0 = T(0), r1 = T(0);
             if (ty == 0) {
                 T gx, gy;
-                pair_force(C, st.px - csx, st.py - csy, st.vx - vsx, st.vy - vsy,
-                           br.r + ro + C.margin, br.ddv, gx, gy);
+                felt = pair_force(C, st.px - csx, st.py - csy, st.vx - vsx, st.vy - vsy,
+                                  br.r + ro + C.margin, br.ddv, gx, gy);
                 f0 = -gx;
                 f1 = -gy;
             } else {
+                felt = true;  // within the shape's bound
                 body_reaction_v<T, T>(C, ty, ro, hx, hy, br.r, br.dd, st.px, st.py, st.vx, st.vy,
                                       csx, csy, B.ca, B.sa, vsx, vsy, B.om, f0, f1, r0, r1);
             }
@@ -730,7 +734,7 @@ __device__ __forceinline__ void body_sum(const Cst<T> &C, const ObTab<T> &tb,
         {
             T acc[3] = {fx, fy, tau};
             const T val[3] = {f0, f1, tq};
-            if (hit && rec && L.any(f0 != T(0) || f1 != T(0))) *hit |= 1ull << (s & 63);
+            if (hit && rec && L.any(felt)) *hit |= 1ull << (s & 63);
             L.template ordered<3>(acc, val, f0 != T(0) || f1 != T(0));
             fx = acc[0];
             fy = acc[1];
@@ -1119,7 +1123,7 @@ __host__ __device__ constexpr size_t body_fwd_lds_total(int PA, int N, size_t ts
 // the lane's agent adjoint is accumulated into `ga`.  ext / cs_in / cs_out / sums are what
 // the forward body_pass of this substep read and wrote: each body's new state is rebuilt
 // from its recorded contact sum, not summed again (NULL cs / sums: recomputed).  `hit`: the
-// shapes that felt a reaction (body_sum); the others' agent terms are zero and are left out.
+// shapes in contact with an agent (body_sum); the others' agent terms are zero and are left out.
 // `obn` (nullable): the state after the substep, read where no clamp asks for the way there.
 // Same order of terms as the oracle's bodies_env_adj.
 template <typename T, typename X, bool SM>

@@ -48,3 +48,22 @@ def test_lane_tape_matches_recompute(E, A, S, extra, world, shapes, dtype):
         for name, x, y in zip(names, runs[0], other):
             assert np.array_equal(x, y), f"{name} differ"
     assert np.abs(runs[0][4]).max() > 0
+
+
+def test_agent_at_the_centre_of_a_shape():
+    """An agent exactly at a round shape's centre exerts no force on it, yet the derivative is
+    the largest a contact has (the offset divided by the contact law's smallest distance): the
+    tape has to name the shape.  No other agent is near the body."""
+    E, A, td = 3, 4, torch.float32
+    s0, acts = _pushers(E, A, 5, spread=0.8)
+    s0[:, :, 0:2] = [[0.0, 0.0], [0.9, 0.9], [-0.9, 0.9], [0.9, -0.9]]
+    runs = []
+    for tape in (True, False):
+        st = make_stepper(nav_agents(A), _world(), 0.05, 2, td, obs=cross_obs(E, (0.0, 0.0)),
+                          n_envs=E)
+        st.use_tape = tape
+        runs.append(hip_body_run(st, s0, acts[:1], td, seed=3)[0])
+    for name, x, y in zip(("agent states", "obstacle states", "d/d pos0", "d/d ob0", "d/d actions"),
+                          *runs):
+        assert np.array_equal(x, y), f"{name} differ"
+    assert np.abs(runs[1][3]).max() > 1e3  # the contact's derivative reaches the body
