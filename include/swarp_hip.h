@@ -351,6 +351,20 @@ int swarp_edge_index(int32_t n_envs, int32_t n_agents, int32_t max_neighbors,
                      const int32_t *idx, const int32_t *cnt, const int64_t *offsets,
                      int64_t n_edges, int64_t *edge_index, void *stream);
 
+/* The same edges without a prefix sum from the caller, in two calls around the allocation of
+ * the result.  Counts are read as min(max(cnt, 0), max_neighbors).
+ * swarp_edge_tiles: the length of `sums` and `host_sums` (at most 1024).
+ * swarp_edge_count: writes the count sums of the agents' tiles to `sums` (device) and
+ * `host_sums` (pinned host memory), waits for the stream and leaves the edge count in the host
+ * value *n_edges.  Not for a stream under capture.
+ * swarp_edge_fill: writes edge_index [2, n_edges] from the same lists and `sums`. */
+int64_t swarp_edge_tiles(int32_t n_envs, int32_t n_agents);
+int swarp_edge_count(int32_t n_envs, int32_t n_agents, int32_t max_neighbors, const int32_t *cnt,
+                     int64_t *sums, int64_t *host_sums, int64_t *n_edges, void *stream);
+int swarp_edge_fill(int32_t n_envs, int32_t n_agents, int32_t max_neighbors, const int32_t *idx,
+                    const int32_t *cnt, const int64_t *sums, int64_t n_edges, int64_t *edge_index,
+                    void *stream);
+
 /* The COO radius graph without any allocation.  No counterpart in the reference: for
  * callers that cannot allocate device memory (code under HIP graph capture, tight
  * serving loops, harnesses that forbid hipMalloc).  Same edges in the same order as

@@ -192,6 +192,17 @@ SIGNATURES = {
          ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p, ctypes.c_void_p],
         ctypes.c_int,
     ),
+    "swarp_edge_tiles": ([ctypes.c_int32, ctypes.c_int32], ctypes.c_int64),
+    "swarp_edge_count": (
+        [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p,
+         ctypes.c_void_p, ctypes.POINTER(ctypes.c_int64), ctypes.c_void_p],
+        ctypes.c_int,
+    ),
+    "swarp_edge_fill": (
+        [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p,
+         ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p, ctypes.c_void_p],
+        ctypes.c_int,
+    ),
     "swarp_edge_index_noalloc": (
         [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p,
          ctypes.c_int64, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p],

@@ -145,9 +145,10 @@ class NeighborGrid:
         self.neighbor_idx = torch.zeros(n_envs, n_agents, max_neighbors, **z)
         self.neighbor_count = torch.zeros(n_envs, n_agents, **z)
         self.neighbor_true_count = torch.zeros(n_envs, n_agents, **z)
-        # edge_index's running sums of the counts: [0, c0, c0 + c1, ...] (the leading
-        # zero is written once, so [:-1] are the exclusive offsets and [-1] the edge count)
-        self._csum = torch.zeros(n_envs * n_agents + 1, device=self.device, dtype=torch.int64)
+        # edge_index's count sums per tile of agents (at most 1024: swarp_edge_tiles), on the
+        # device and, once edge_index was called, in pinned host memory
+        self._tile_sums = torch.zeros(1024, device=self.device, dtype=torch.int64)
+        self._host_sums = None
         self.build_count = 0
         self.built_version = -1
         # the batch-reduced grid frame (origin x, y, cell size) of the last build
@@ -240,16 +241,18 @@ class NeighborGrid:
         cnt = self.neighbor_count.reshape(-1)
         if cnt.numel() == 0:
             return torch.empty(2, 0, device=self.device, dtype=torch.int64)
-        torch.cumsum(cnt, 0, dtype=torch.int64, out=self._csum[1:])
-        n_edges = int(self._csum[-1].item())
-        out = torch.empty(2, n_edges, device=self.device, dtype=torch.int64)
-        if n_edges == 0:
-            return out
-        offsets = self._csum[:-1]
+        if self._host_sums is None:
+            self._host_sums = torch.zeros(1024, dtype=torch.int64, pin_memory=True)
         lib = _lib.load()
-        stream = _lib.stream_of(out.device)
-        _lib.check(lib.swarp_edge_index(
+        stream = _lib.stream_of(cnt.device)
+        n = ctypes.c_int64()
+        _lib.check(lib.swarp_edge_count(
+            self.n_envs, self.n_agents, self.max_neighbors, cnt.data_ptr(),
+            self._tile_sums.data_ptr(), self._host_sums.data_ptr(), ctypes.byref(n), stream,
+        ))
+        out = torch.empty(2, n.value, device=self.device, dtype=torch.int64)
+        _lib.check(lib.swarp_edge_fill(
             self.n_envs, self.n_agents, self.max_neighbors, self.neighbor_idx.data_ptr(),
-            self.neighbor_count.data_ptr(), offsets.data_ptr(), n_edges, out.data_ptr(), stream,
+            cnt.data_ptr(), self._tile_sums.data_ptr(), n.value, out.data_ptr(), stream,
         ))
         return out

@@ -1,5 +1,5 @@
-"""``swarp_edge_index_noalloc`` (the allocation-free COO radius graph) against the existing
-entry point ``swarp_edge_index`` (through ``NeighborGrid.edge_index``), both called
+"""``swarp_edge_index_noalloc`` (the allocation-free COO radius graph) against
+``NeighborGrid.edge_index`` (``swarp_edge_count`` / ``swarp_edge_fill``), both called
 through the C ABI: identical edges in identical order, on two calls in a row with the
 second one smaller (the file-scope scratch keeps the first call's partial sums), a
 capacity below the edge count (edges past it dropped, the true count still reported),
@@ -43,7 +43,7 @@ def _noalloc(g, E, A, K, capacity):
 def test_two_calls_match_existing_entry_point(shapes):
     for k, (E, A, r, K, spread) in enumerate(shapes):
         g = _lists(E, A, r, K, spread, seed=10 + k)
-        ref = g.edge_index()  # swarp_edge_index with torch's prefix sums
+        ref = g.edge_index()
         cap = E * A * K
         out, n = _noalloc(g, E, A, K, cap)
         m = ref.shape[1]
