@@ -160,7 +160,9 @@ template <typename T> __device__ __forceinline__ int near_axis(T p, T o, T i, in
 
 // The candidates of one agent once the sort is complete, as they come.  Returns how many
 // there are; those past the list's room are not kept.  A started word is filled up with the
-// agent's own id, which every reader skips.
+// agent's own id, which every reader skips.  A word is put together in a register and stored
+// once: its ids stored one by one as 16-bit values would be accesses of another type than the
+// word's, which the compiler may order as it likes.
 template <typename T>
 __device__ __forceinline__ int near_find(const WideLds<T> &W, const NearLds<T> &N,
                                          const NearGrid<T> &H, int i, T px, T py)
@@ -177,7 +179,8 @@ __device__ __forceinline__ int near_find(const WideLds<T> &W, const NearLds<T> &
         q1[k] = in ? N.start[row + x1] : q0[k];
     }
     int n = 0;
-    uint16_t *const mine = (uint16_t *)(N.cand + i);
+    const uint64_t own = (uint64_t)i * 0x0001000100010001ull;
+    uint64_t word = own;
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
         for (int q = q0[k]; q < q1[k]; q += 4) {
@@ -194,14 +197,16 @@ __device__ __forceinline__ int near_find(const WideLds<T> &W, const NearLds<T> &
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
                 if (!hit[u]) continue;
-                if (n < N.cap) {
-                    if ((n & 3) == 0) N.cand[(n >> 2) * N.AP + i] = (uint64_t)i * 0x0001000100010001ull;
-                    mine[(n >> 2) * N.AP * 4 + (n & 3)] = (uint16_t)j[u];
+                word ^= (uint64_t)(uint32_t)(j[u] ^ i) << (16 * (n & 3));
+                if ((n & 3) == 3) {
+                    if (n < N.cap) N.cand[(n >> 2) * N.AP + i] = word;
+                    word = own;
                 }
                 ++n;
             }
         }
     }
+    if ((n & 3) != 0 && n < N.cap) N.cand[(n >> 2) * N.AP + i] = word;
     return n;
 }
 
@@ -308,7 +313,8 @@ __device__ __forceinline__ void near_forces(const Cst<T> &C, const WideLds<T> &W
     for (int c = 0; c < listed && c < C.K; ++c) {
         int best = CUT_ALL;
         for (int e = 0; e < n; ++e) {
-            const int j = ((const uint16_t *)(N.cand + (e >> 2) * N.AP + L.i))[e & 3];
+            const uint64_t w = N.cand[(e >> 2) * N.AP + L.i];
+            const int j = (int)((uint32_t)(w >> (16 * (e & 3))) & 0xffffu);
             int key;
             const bool in = near_key<T, GRID>(C, W, N, L.i, me, j, st.px - W.px[j],
                                               st.py - W.py[j], key);

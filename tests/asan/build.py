@@ -82,6 +82,28 @@ def build(jobs: int = 8) -> Path:
     return EXE
 
 
+NEAR = ["-std=c++17", "-ffp-contract=off", "-pthread", "-w", f"-I{HERE / 'emu'}", f"-I{SRC}",
+        str(HERE / "near.cpp")]
+CLANG = Path("/opt/rocm/llvm/bin/clang++")
+
+
+def build_near(typed: bool) -> Path | None:
+    """tests/asan/_build/near: near.cpp, plain (g++ -O2) or under clang's type sanitizer; None
+    where this toolchain has none."""
+    OUT.mkdir(exist_ok=True)
+    stage()
+    exe = OUT / ("near_typed" if typed else "near")
+    if typed and not CLANG.exists():
+        return None
+    cc = [str(CLANG), "-O1", "-g", "-fsanitize=type"] if typed else ["g++", "-O2"]
+    r = subprocess.run([*cc, *NEAR, "-o", str(exe)], capture_output=True, text=True)
+    if typed and r.returncode and "clang_rt.tysan" in r.stderr:
+        return None
+    if r.returncode:
+        raise RuntimeError("near build failed:\n" + (r.stdout + r.stderr)[-6000:])
+    return exe
+
+
 if __name__ == "__main__":
     print(build())
     sys.exit(0)
