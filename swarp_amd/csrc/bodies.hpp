@@ -44,6 +44,27 @@ template <typename T> struct ObTab {
     int cache;   // backward: 1 keeps each substep's body cos / sin and contact sums in LDS
 };
 
+// The tables with each pointer in a register pair of its own.  The compiler reads them from the
+// kernel arguments sixteen registers at a time and, where scalar registers are short, spills
+// and restores all sixteen as one value in every block that needs a single pointer.
+template <typename P> __device__ __forceinline__ P own_pair(P p)
+{
+    asm volatile("" : "+s"(p));
+    return p;
+}
+template <typename T> __device__ __forceinline__ ObTab<T> apart(ObTab<T> t)
+{
+    t.rad = own_pair(t.rad);
+    t.half = own_pair(t.half);
+    t.mass = own_pair(t.mass);
+    t.inertia = own_pair(t.inertia);
+    t.off = own_pair(t.off);
+    t.type = own_pair(t.type);
+    t.kind = own_pair(t.kind);
+    t.body = own_pair(t.body);
+    return t;
+}
+
 // Obstacle-state inputs / outputs of a rollout.
 template <typename T> struct ObIO {
     const T *ob0;       // [E, 12N] state entering the rollout
@@ -1126,8 +1147,13 @@ __host__ __device__ constexpr size_t body_fwd_lds_total(int PA, int N, size_t ts
 // shapes in contact with an agent (body_sum); the others' agent terms are zero and are left out.
 // `obn` (nullable): the state after the substep, read where no clamp asks for the way there.
 // Same order of terms as the oracle's bodies_env_adj.
+// The pairs of shapes bound it where an env holds many.  In the general instances (SM false) that
+// loop issued 16 register moves a block for the tables' spilled pointers: 2000 envs x 64 agents,
+// 100 shapes of 20 bodies, 4 steps of 2 substeps, backward 57.4 -> 40.5 ms with the pointers
+// apart.  The profile's instances hold few enough scalars: 40 shapes, 3.38 ms as they are and
+// 3.58 apart.
 template <typename T, typename X, bool SM>
-__device__ __forceinline__ void body_pass_adj(const Cst<T> &C, const ObTab<T> &tb,
+__device__ __forceinline__ void body_pass_adj(const Cst<T> &C, const ObTab<T> &tab,
                                               const ShapeSets<T, SM> &SS,
                                               const X &L, const BodyRow<T> &br,
                                               const St<T> &st, const T *obc, const T *gout,
@@ -1135,6 +1161,7 @@ __device__ __forceinline__ void body_pass_adj(const Cst<T> &C, const ObTab<T> &t
                                               const T *cs_out, const T *sums,
                                               uint64_t hit = ~0ull, const T *obn = nullptr)
 {
+    const ObTab<T> tb = SM ? tab : apart(tab);
     const int N = tb.N;
     // pass-through of everything the pass does not rewrite
     for (int q = L.me(); q < OB_W * N; q += L.stride()) {
