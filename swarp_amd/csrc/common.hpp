@@ -338,82 +338,91 @@ template <typename M> __device__ __forceinline__ M cap_list(M incl, int K)
     return incl ^ rest;
 }
 
-// Padded list rows leave a wave straight from the lists' masks.  A row of K 4-byte slots written
-// to LDS by its lane, slot by slot, puts every lane's k-th word in one bank when K is a
-// multiple of 32 and a few otherwise, and holds 256 K bytes of LDS; instead each row's mask and
-// its first four members (a byte each: most rows hold no more) go to LDS, and the wave's lanes
-// form the output 16 bytes at a time in memory order.
+// Padded list rows leave a wave through LDS as packed ids.  A row of K 4-byte slots written
+// there by its lane, slot by slot, holds 256 K bytes of LDS a wave; instead a row's members are
+// packed a byte each (an id is below 64), as far as it has members and at an odd word stride, and
+// the wave's lanes form the output 16 bytes at a time in memory order.  Forming each piece from
+// the row's mask, by clearing the bits before it, took full rows longer than whole slots do.
+// 16000 envs x 64 agents, us, whole slots / from masks / packed: every other agent listed, K = 64
+// 59 / 143 / 46, K = 32 33 / 55 / 31; rows of less than one member, 57 / 40 / 41 and 30 / 24 / 23.
 //   row_put   one lane's row r
 //   rows_out  `n` consecutive rows from row r0 to dst
-template <typename M> struct RowLds {
-    M mask[64];
-    uint32_t four[64];
+struct RowLds {
+    uint32_t *word, *cnt;  // [64][stride] packed members, [64] how many
+    int stride;
 };
 
-template <typename M> __device__ __forceinline__ void row_put(RowLds<M> &R, int r, M m)
+// Words from one row to the next for rows of at most K of PA agents, and the LDS they take.
+__host__ __device__ inline int row_stride(int PA, int K) { return ((K < PA ? K : PA) + 3) / 4 | 1; }
+__host__ __device__ inline size_t row_lds_bytes(int PA, int K)
 {
-    R.mask[r] = m;
-    uint32_t w = 0;
+    return (size_t)64 * (row_stride(PA, K) + 1) * sizeof(uint32_t);
+}
+
+__device__ __forceinline__ RowLds row_lds(void *smem, int PA, int K)
+{
+    const int s = row_stride(PA, K);
+    return {(uint32_t *)smem, (uint32_t *)smem + 64 * s, s};
+}
+
+template <typename M> __device__ __forceinline__ void row_put(const RowLds &R, int r, M m)
+{
+    R.cnt[r] = (uint32_t)m_popc(m);
+    uint32_t *p = R.word + r * R.stride;
+    do {
+        uint32_t w = 0;
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        if (m) w |= (uint32_t)m_ctz(m) << (8 * k);
-        m &= m - 1;
-    }
-    R.four[r] = w;
+        for (int k = 0; k < 4; ++k) {
+            if (m) w |= (uint32_t)m_ctz(m) << (8 * k);
+            m &= m - 1;
+        }
+        *p++ = w;
+    } while (m);
 }
 
-template <typename M> __device__ __forceinline__ int32_t row_slot(const RowLds<M> &R, int r, int k)
+// Slots 4 c .. 4 c + 3 of row r, packed (those past the members are 0).
+__device__ __forceinline__ uint32_t row_piece(const RowLds &R, int r, int c)
 {
-    if (k < 4) return (int32_t)((R.four[r] >> (8 * k)) & 0xffu);
-    M m = R.mask[r];
-    if (k >= m_popc(m)) return 0;
-    for (int q = 0; q < k; ++q) m &= m - 1;
-    return m_ctz(m);
+    const uint32_t n = R.cnt[r], w = R.word[r * R.stride + (c < R.stride ? c : 0)];
+    return (uint32_t)(4 * c) < n ? w : 0u;
 }
 
-template <typename M>
-__device__ __forceinline__ void rows_out(int32_t *dst, const RowLds<M> &R, int r0, int n, int K,
+__device__ __forceinline__ int4 row_ids(uint32_t w)
+{
+    return make_int4((int)(w & 0xffu), (int)((w >> 8) & 0xffu), (int)((w >> 16) & 0xffu), (int)(w >> 24));
+}
+
+__device__ __forceinline__ void rows_out(int32_t *dst, const RowLds &R, int r0, int n, int K,
                                          int lane)
 {
-    const int per = (K & 3) == 0 && ((uintptr_t)dst & 15u) == 0u ? 4 : 1;  // slots per store
-    const int P = K / per, total = n * P;  // stores per row, and in all
-    int r = r0 + lane / P, c = lane % P;
-    const int dr = 64 / P, dc = 64 % P;
-    if (per == 4) {
-        for (int q = lane; q < total; q += 64) {
-            int4 v = make_int4(0, 0, 0, 0);
-            if (c == 0) {
-                const uint32_t w = R.four[r];
-                v = make_int4(w & 0xffu, (w >> 8) & 0xffu, (w >> 16) & 0xffu, w >> 24);
-            } else {
-                M m = R.mask[r];
-                if (4 * c < m_popc(m)) {
-                    for (int k = 0; k < 4 * c; ++k) m &= m - 1;
-                    int e[4];
-#pragma unroll
-                    for (int k = 0; k < 4; ++k) {
-                        e[k] = m ? m_ctz(m) : 0;
-                        m &= m - 1;
-                    }
-                    v = make_int4(e[0], e[1], e[2], e[3]);
-                }
-            }
-            ((int4 *)dst)[q] = v;
-            r += dr;
-            c += dc;
-            if (c >= P) {
-                c -= P;
-                ++r;
-            }
+    const int total = n * K;
+    const bool wide = ((uintptr_t)dst & 15u) == 0u && (total & 3) == 0 && K >= 4;
+    const int per = wide ? 4 : 1, step = 64 * per;  // slots per store
+    // quotients of at most 256 by K: (x + 1/2) / K is further from a whole number than the
+    // reciprocal is off, so its floor is the quotient (two integer divisions took a tenth of
+    // the build of short rows)
+    const float inv = __builtin_amdgcn_rcpf((float)K);
+    const int dr = (int)(((float)step + 0.5f) * inv), dk = step - dr * K;
+    int r = (int)(((float)(lane * per) + 0.5f) * inv), k = lane * per - r * K;
+    r += r0;
+    for (int q = lane * per; q < total; q += step) {
+        const uint32_t w = row_piece(R, r, k >> 2);
+        if (wide && (K & 3) == 0) {
+            *(int4 *)(dst + q) = row_ids(w);
+        } else if (wide) {
+            // four slots from within a piece: of two pieces of this row and, past its end, the
+            // first of the next (K >= 4: of no third row)
+            const int sh = 8 * (k & 3), left = K - k;
+            uint32_t v = (uint32_t)((((uint64_t)row_piece(R, r, (k >> 2) + 1) << 32) | w) >> sh);
+            if (left < 4) v = (v & ((1u << (8 * left)) - 1u)) | R.word[(r + 1) * R.stride] << (8 * left);
+            *(int4 *)(dst + q) = row_ids(v);
+        } else {
+            dst[q] = (int32_t)((w >> (8 * (k & 3))) & 0xffu);
         }
-        return;
-    }
-    for (int q = lane; q < total; q += 64) {
-        dst[q] = row_slot(R, r, c);
         r += dr;
-        c += dc;
-        if (c >= P) {
-            c -= P;
+        k += dk;
+        if (k >= K) {
+            k -= K;
             ++r;
         }
     }

@@ -11,8 +11,8 @@
 // Layout: one lane per (env, agent) as in the step kernels -- an env is PA consecutive
 // lanes of a wave64, so the env's lists and its reward reduction stay inside the wave
 // (positions and per-agent terms in LDS, no global atomics).  Observation rows are
-// assembled in LDS and leave as contiguous, coalesced stores when they fit; list rows leave
-// from their masks (rows_out).  Writing bounds the pass (319 MB at 16000 envs x 64 agents, of
+// assembled in LDS and leave as contiguous, coalesced stores when they fit; then the list rows
+// leave through the same LDS, packed (rows_out).  Writing bounds the pass (319 MB at 16000 envs x 64 agents, of
 // which 131 MB are list slots); with the list rows staged in LDS as well, their bank conflicts
 // and the 15 KB a wave held did: 102 -> 51 us.
 // Instantiated by k_nav.hip.
@@ -56,10 +56,10 @@ __global__ __launch_bounds__(64) void k_nav(const Cst<T> C, const NavArgs<T> g)
     typedef typename MaskT<PA>::type M;
     __shared__ T lx[64], ly[64], lvx[64], lvy[64], lra[64], lsh[64];
     __shared__ int log_[64];
-    __shared__ RowLds<M> rows;
     extern __shared__ __align__(16) unsigned char nav_dyn[];
-    // staged observation rows [EPW * A][W]
-    T *row_lds = reinterpret_cast<T *>(nav_dyn);
+    // staged observation rows [EPW * A][W] and, once those have left, the list rows
+    T *obs_lds = reinterpret_cast<T *>(nav_dyn);
+    const RowLds rows = row_lds(nav_dyn, PA, C.K);
 
     const int lane = threadIdx.x, agent = lane % PA, base = lane - agent;
     const int env = blockIdx.x * (64 / PA) + lane / PA;
@@ -98,7 +98,6 @@ __global__ __launch_bounds__(64) void k_nav(const Cst<T> C, const NavArgs<T> g)
     const M incl = scan_all<T, PA>(lx, ly, base, C.A, agent, px, py, C.t_nbr, C.t_nbr, cd);
     const M m = cap_list(incl, C.K);
     const int n = m_popc(m);
-    if (real) row_put(rows, row, m);
     if (work) {
         g.cnt[i] = n;
         if (g.tru) g.tru[i] = m_popc(incl);
@@ -132,7 +131,7 @@ __global__ __launch_bounds__(64) void k_nav(const Cst<T> C, const NavArgs<T> g)
     // observation row (_obs_row, :41-89)
     const int W = g.W, KO = g.k_obs;
     {
-        T *dst = g.stage ? row_lds + (size_t)row * W : g.obs + i * W;
+        T *dst = g.stage ? obs_lds + (size_t)row * W : g.obs + i * W;
         const bool put = g.stage ? real : work;
         if (put) {
             dst[0] = px;
@@ -195,11 +194,17 @@ __global__ __launch_bounds__(64) void k_nav(const Cst<T> C, const NavArgs<T> g)
         const int env0 = blockIdx.x * (64 / PA);
         const int n_env = min(64 / PA, C.E - env0);
         const int blocks = g.full_pass != 0 ? 1 : n_env, per = g.full_pass != 0 ? n_env * C.A : C.A;
-        for (int e = 0; e < blocks; ++e) {
+        for (int e = 0; e < blocks && g.stage; ++e) {
             if (g.full_pass == 0 && !(g.rmask != nullptr && g.rmask[env0 + e] != 0)) continue;
             const size_t first = (size_t)env0 * C.A + (size_t)e * per;
-            if (g.stage) wave_copy(g.obs + first * W, row_lds + (size_t)e * per * W, per * W, lane);
-            rows_out(g.idx + first * C.K, rows, e * per, per, C.K, lane);
+            wave_copy(g.obs + first * W, obs_lds + (size_t)e * per * W, per * W, lane);
+        }
+        wave_lds_sync();  // (the workgroup is this one wave)
+        if (real) row_put(rows, row, m);
+        wave_lds_sync();
+        for (int e = 0; e < blocks; ++e) {
+            if (g.full_pass == 0 && !(g.rmask != nullptr && g.rmask[env0 + e] != 0)) continue;
+            rows_out(g.idx + ((size_t)env0 * C.A + (size_t)e * per) * C.K, rows, e * per, per, C.K, lane);
         }
     }
 

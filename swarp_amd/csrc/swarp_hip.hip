@@ -762,8 +762,9 @@ template <typename T> static int nav_obs(const swarp_desc_t *d, const swarp_nav_
     g.max_steps = v->max_steps;
     const size_t lds = (size_t)64 * g.W * sizeof(T);
     g.stage = lds <= 48 * 1024 ? 1 : 0;  // observation rows leave through LDS when they fit
-    const unsigned dyn = g.stage ? (unsigned)lds : 0u;
     const int PA = pad_agents(d->n_agents);
+    const size_t rows = row_lds_bytes(PA, C.K);  // the list rows, in the same place
+    const unsigned dyn = (unsigned)(g.stage && lds > rows ? lds : rows);
     launch_nav<T>(PA, C, g, dyn, st);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(hipGetErrorString(e));

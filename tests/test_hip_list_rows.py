@@ -25,6 +25,16 @@ pytestmark = pytest.mark.gpu
     (1, 700, 33, 0.3, 0),    # grid order
     (1, 520, 520, 1.0, 0),   # rows too long to be staged
     (1, 3000, 60, 0.1, 0),
+    # one wave's rows: whole slots up to 16 of them, packed ids beyond
+    (3, 64, 16, 3.0, 0),     # the longest whole rows, full
+    (3, 64, 15, 3.0, 0),
+    (4, 64, 17, 3.0, 0),     # packed, a store from two pieces and, past the end, the next row
+    (4, 64, 18, 0.6, 0),
+    (4, 61, 19, 3.0, 0),     # slots of the wave not a multiple of 4
+    (5, 40, 33, 3.0, 2),     # packed, a 4-byte boundary
+    (6, 13, 40, 3.0, 0),     # more slots than agents
+    (7, 4, 20, 3.0, 0),
+    (1, 64, 300, 3.0, 0),    # more slots than a store step
 ])
 def test_rows(E, A, K, r, shift):
     rng = np.random.default_rng(A + K)
