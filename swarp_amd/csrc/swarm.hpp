@@ -14,8 +14,9 @@
 // agents in arrival order and candidates come as found, but a list is taken from them by key
 // -- the index, or for the uniform grid (slot of the 3x3 block, index), which orders as (slot,
 // rank in the cell) does -- so no result depends on it.  An env that overflows its candidate
-// lists takes a quarter of the skin, and overflowing that too falls back, for the rest of the
-// rollout, to wide.hpp's traversal of the whole list at every substep.
+// lists takes a quarter of the skin (where that pays, see NEAR_FULL) and else falls back, for the
+// rest of the rollout, to wide.hpp's traversal of the whole list at every substep: a search in
+// vain dearer than that traversal alone, which is 2 to 8 % of a crowded rollout.
 //
 // Tape.  The forward leaves each substep's total force and the agents it touched (up to
 // NEAR_TOUCH ids); the backward then integrates to the substeps' inputs with the recorded
@@ -28,8 +29,8 @@
 // them), not bandwidth and not issue.  Measured (MI355X, holonomic agents between walls),
 // forward / backward, before (every pair tested at every substep, the backward recomputing
 // the lists of S (S + 1) / 2 substeps a step) and now: 500 envs x 200 agents, 8 steps of 4
-// substeps 595 / 2326 -> 141 / 120 us; 48 x 2000, uniform grid, 8 steps of 2 substeps 519 /
-// 1402 -> 226 / 157 us.  Candidates through chains of hashed cells instead of sorted runs
+// substeps 595 / 2326 -> 129 / 121 us; 48 x 2000, uniform grid, 8 steps of 2 substeps 519 /
+// 1402 -> 213 / 169 us.  Candidates through chains of hashed cells instead of sorted runs
 // took 310 and 465 us forward: a chain is a dependent LDS read per agent of the block.
 #pragma once
 #include "wide.hpp"
@@ -39,6 +40,12 @@ namespace swarp {
 constexpr int NEAR_MAX = 16;   // candidates an agent keeps (fewer where the LDS is short)
 constexpr int NEAR_TOUCH = 8;  // touching agents a tape record holds
 constexpr uint32_t NEAR_NONE = 0xffffu, NEAR_SLOW = 0xfffeu;
+
+// Index-ordered envs of up to this many agents whose candidates overflow take no quarter of the
+// skin: their full traversal is short.  Forward without gradient, 16 substeps, 60 agents per unit
+// area, us, a quarter / the full traversal: 857 envs x 70 agents 262 / 202, 461 x 130 304 / 290,
+// and at 15 per unit area and more agents 300 x 200 152 / 352, 60 x 1000 171 / 1833.
+constexpr int NEAR_FULL = 128;
 
 // Most cells per axis of the search: about four cells per agent slot (fewer are used where
 // the skin radius asks for wider ones; the scan covers those used).
@@ -124,7 +131,7 @@ template <typename T> struct NearGrid {
     T t_skin, half2;   // squared skin radius, squared displacement the candidates bear
 };
 
-// Cells for a skin of `part` of the launch's (1 or 1 / 4) over a box.  The cells are wider than
+// Cells for a skin of `part` (0 .. 1) of the launch's over a box.  The cells are wider than
 // the skin radius by 1/16, far above the roundings of (p - o) * i below 64 cells, so agents
 // within the skin radius of each other land at most one cell apart.
 template <typename T>
@@ -204,6 +211,7 @@ __device__ __forceinline__ int near_find(const WideLds<T> &W, const NearLds<T> &
                 }
                 ++n;
             }
+            if (n > N.cap) return n;  // the env gives these up
         }
     }
     if ((n & 3) != 0 && n < N.cap) N.cand[(n >> 2) * N.AP + i] = word;
@@ -233,17 +241,18 @@ struct NearRec {
     __device__ __forceinline__ bool second() const { return !slow && n >= 4; }
 };
 
-// Contact force of agent j on the lane's agent, added and recorded.
+// Contact force of agent j on the lane's agent, added and (`keep`: there is a tape) recorded.
 template <typename T>
 __device__ __forceinline__ void near_pair(const Cst<T> &C, const WideLds<T> &W, const WLane<T> &L,
-                                          const St<T> &st, int j, T &fx, T &fy, NearRec &rec)
+                                          const St<T> &st, int j, T &fx, T &fy, NearRec &rec,
+                                          bool keep)
 {
     T gx, gy;
     if (pair_force(C, st.px - W.px[j], st.py - W.py[j], st.vx - W.vx[j], st.vy - W.vy[j],
                    L.pr.radius + W.rad[j] + C.margin, L.ddv, gx, gy)) {
         fx += gx;  // apart, a pair adds exactly +0
         fy += gy;
-        rec.push(j);
+        if (keep) rec.push(j);
     }
 }
 
@@ -265,78 +274,88 @@ __device__ __forceinline__ bool near_key(const Cst<T> &C, const WideLds<T> &W, c
     return in;
 }
 
-// Contact forces of an agent from its `n` candidates: its capped list in list order.  One
-// pass counts the members and keeps the keys of the first NK that may touch; where the cap
-// does not bite and no more may touch those are the list's whole force.  Otherwise the
-// members are taken one after the other by ascending key.
+// Contact forces of an agent from its `n` candidates: its capped list in list order.  A pass
+// over them counts the members and keeps the NK smallest keys above `last` of those that may
+// touch: where the cap does not bite and no more may touch, those are the list's whole force.
+// Otherwise pass after pass takes the next NK of the close ones or, where the cap bites, of all
+// members.  (Taken one at a time, a pass for each, crowded agents bound the substep: 461 envs x
+// 130 agents, 60 per unit area, 16 substeps forward 515 us, now 290, the full traversal 270; 857 x
+// 70, 30 per unit area, 335, 188 and 175.)
 template <typename T, bool GRID>
 __device__ __forceinline__ void near_forces(const Cst<T> &C, const WideLds<T> &W,
                                             const NearLds<T> &N, const WLane<T> &L,
-                                            const St<T> &st, int n, T &fx, T &fy, NearRec &rec)
+                                            const St<T> &st, int n, T &fx, T &fy, NearRec &rec,
+                                            bool keep)
 {
     constexpr int NK = 4;
     const uint32_t me = GRID ? N.cell[L.i] : 0u;
-    int listed = 0, near = 0;
-    int ks[NK];
+    int listed = 0, near = 0, ks[NK];
+    auto pass = [&](bool all, int last) {
+        listed = near = 0;
 #pragma unroll
-    for (int c = 0; c < NK; ++c) ks[c] = CUT_ALL;
-    for (int e = 0; e < n; e += 4) {
-        const uint64_t w = N.cand[(e >> 2) * N.AP + L.i];
+        for (int c = 0; c < NK; ++c) ks[c] = CUT_ALL;
+        for (int e = 0; e < n; e += 4) {
+            const uint64_t w = N.cand[(e >> 2) * N.AP + L.i];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int j = (int)((uint32_t)(w >> (16 * u)) & 0xffffu);
-            const T dx = st.px - W.px[j], dy = st.py - W.py[j];
-            int key;
-            const bool in = near_key<T, GRID>(C, W, N, L.i, me, j, dx, dy, key);
-            const bool close = in && !pair_apart(dx, dy, L.pr.radius + W.rad[j] + C.margin);
-            listed += in ? 1 : 0;
-            near += close ? 1 : 0;
-            int x = close ? key : CUT_ALL;
+            for (int u = 0; u < 4; ++u) {
+                const int j = (int)((uint32_t)(w >> (16 * u)) & 0xffffu);
+                const T dx = st.px - W.px[j], dy = st.py - W.py[j];
+                int key;
+                const bool in = near_key<T, GRID>(C, W, N, L.i, me, j, dx, dy, key);
+                const bool close = in && !pair_apart(dx, dy, L.pr.radius + W.rad[j] + C.margin);
+                listed += in ? 1 : 0;
+                near += close ? 1 : 0;
+                int x = (all ? in : close) && key > last ? key : CUT_ALL;
 #pragma unroll
-            for (int c = 0; c < NK; ++c) {
-                const int lo = x < ks[c] ? x : ks[c];
-                x = x < ks[c] ? ks[c] : x;
-                ks[c] = lo;
+                for (int c = 0; c < NK; ++c) {
+                    const int lo = x < ks[c] ? x : ks[c];
+                    x = x < ks[c] ? ks[c] : x;
+                    ks[c] = lo;
+                }
             }
         }
-    }
-    if (listed <= C.K && near <= NK) {
+    };
+    pass(false, -1);
+    const bool cut = listed > C.K;
+    rec.slow = cut;
+    if (!cut && near <= NK) {
         for (int c = 0; c < near; ++c) {
-            near_pair(C, W, L, st, GRID ? ks[0] % WIDE_MAX_AGENTS : ks[0], fx, fy, rec);
+            near_pair(C, W, L, st, GRID ? ks[0] % WIDE_MAX_AGENTS : ks[0], fx, fy, rec, keep);
 #pragma unroll
             for (int k = 0; k + 1 < NK; ++k) ks[k] = ks[k + 1];
         }
         return;
     }
-    rec.slow = listed > C.K;
-    int last = -1;
-    for (int c = 0; c < listed && c < C.K; ++c) {
-        int best = CUT_ALL;
-        for (int e = 0; e < n; ++e) {
-            const uint64_t w = N.cand[(e >> 2) * N.AP + L.i];
-            const int j = (int)((uint32_t)(w >> (16 * (e & 3))) & 0xffffu);
-            int key;
-            const bool in = near_key<T, GRID>(C, W, N, L.i, me, j, st.px - W.px[j],
-                                              st.py - W.py[j], key);
-            if (in && key > last && key < best) best = key;
+    int left = cut ? C.K : near;
+    if (cut) pass(true, -1);
+    for (;;) {
+        const int last = ks[NK - 1];
+#pragma unroll 1
+        for (int c = 0; c < NK && c < left; ++c) {
+            near_pair(C, W, L, st, GRID ? ks[0] % WIDE_MAX_AGENTS : ks[0], fx, fy, rec, keep);
+#pragma unroll
+            for (int k = 0; k + 1 < NK; ++k) ks[k] = ks[k + 1];
         }
-        last = best;
-        near_pair(C, W, L, st, GRID ? best % WIDE_MAX_AGENTS : best, fx, fy, rec);
+        left -= NK;
+        if (left <= 0) break;
+        pass(cut, last);
     }
 }
 
-// The same from the full traversal.
-template <typename T, bool GRID>
+// The same from the full traversal.  KEEP is compiled in: in this pair loop the record costs a
+// rollout without a tape where it is only branched around (461 envs x 130 agents, 60 per unit
+// area, neighbours within 0.3, 64 substeps: 1470 us recorded, 1388 branched around, 1345).
+template <typename T, bool GRID, bool KEEP>
 __device__ __forceinline__ void full_forces(const Cst<T> &C, const WideLds<T> &W,
                                             const GridFrame<T> &G, const WLane<T> &L,
                                             const St<T> &st, T &fx, T &fy, NearRec &rec)
 {
     int listed = 0;
     visit_list<T, GRID>(W, C.A, G, L.i, st.px, st.py, C.t_nbr, C.K, false, [&](int j, int32_t) {
-        near_pair(C, W, L, st, j, fx, fy, rec);
+        near_pair(C, W, L, st, j, fx, fy, rec, KEEP);
         ++listed;
     });
-    if (listed >= C.K) rec.slow = true;  // maybe truncated
+    if (KEEP && listed >= C.K) rec.slow = true;  // maybe truncated
 }
 
 template <typename T, bool DRONE, bool GRID, int APT, unsigned F>
@@ -374,8 +393,14 @@ __global__ __launch_bounds__(1024) void k_swarm_fwd(const Cst<T> Cin, const Args
         for (int w = 0; w < (int)blockDim.x / 64; ++w)
             box_join(box, Box4<T>{red[4 * w], red[4 * w + 1], red[4 * w + 2], red[4 * w + 3]});
     }
-    NearGrid<T> H = near_grid(C, box, T(1), AP);
-    bool whole = true;         // the whole skin, not a quarter of it
+    const bool taped = g.fsum != nullptr;
+    // The skin bears two steps' motion, or what a shorter rollout's own substeps need (none for
+    // a single one: 200 envs x 300 agents, 15 per unit area, neighbours within 0.3, one substep
+    // 68 us with the whole skin, 34 without, 48 by the full traversal).
+    const int moves = g.nsteps * C.S - 1;
+    const T part = moves < 2 * C.S ? T(moves) / T(2 * C.S) : T(1);
+    NearGrid<T> H = near_grid(C, box, part, AP);
+    bool whole = moves > 0 && (GRID || C.A > NEAR_FULL);  // a quarter is left to take
     bool dense = N.cap == 0;   // the full traversal   (both the same in every thread)
     T rx[APT], ry[APT];        // where the candidates were found
     int nc[APT];               // how many there are
@@ -446,7 +471,7 @@ __global__ __launch_bounds__(1024) void k_swarm_fwd(const Cst<T> Cin, const Args
                         __syncthreads();  // before the sort, or all its LDS, is used again
                         if (whole) {
                             whole = false;
-                            H = near_grid(C, box, T(0.25), AP);
+                            H = near_grid(C, box, T(0.25) * part, AP);
                             for (int c = threadIdx.x; c < H.nx * H.ny; c += blockDim.x) N.start[c] = 0;
                             __syncthreads();
                         } else {
@@ -461,14 +486,18 @@ __global__ __launch_bounds__(1024) void k_swarm_fwd(const Cst<T> Cin, const Args
                     T fx = T(0), fy = T(0);
                     NearRec rec;
                     if (C.collisions && L[k].active) {
-                        if (dense) full_forces<T, GRID>(C, W, G, L[k], st[k], fx, fy, rec);
-                        else near_forces<T, GRID>(C, W, N, L[k], st[k], nc[k], fx, fy, rec);
+                        if (!dense)
+                            near_forces<T, GRID>(C, W, N, L[k], st[k], nc[k], fx, fy, rec, taped);
+                        else if (taped)
+                            full_forces<T, GRID, true>(C, W, G, L[k], st[k], fx, fy, rec);
+                        else
+                            full_forces<T, GRID, false>(C, W, G, L[k], st[k], fx, fy, rec);
                     }
                     T sx, sy;
                     wide_static_forces(C, g, L[k], st[k], sx, sy);
                     Fx[k] = fx + sx;
                     Fy[k] = fy + sy;
-                    if (g.fsum && L[k].active) {
+                    if (taped && L[k].active) {
                         const size_t q = ((size_t)t * C.S + s) * EA + L[k].idx;
                         g.fsum[2 * q] = Fx[k];
                         g.fsum[2 * q + 1] = Fy[k];

@@ -40,13 +40,14 @@ template <typename T> int check(int A, int near, int K)
     L.ddv = divisor(T(1), true);
     St<T> st;
     st_zero(st);
-    int bad = near_find(W, N, H, 0, st.px, st.py) != near;
+    const int found = near_find(W, N, H, 0, st.px, st.py);
+    int bad = near > N.cap ? found <= N.cap : found != near;  // (it stops once they overflow)
     for (int e = 0; e < near && e < N.cap; ++e)
         bad += (int)(N.cand[(e >> 2) * AP] >> (16 * (e & 3)) & 0xffffu) != near - e;
     if (near > N.cap) return bad;
     T fx = T(0), fy = T(0);
     NearRec rec;
-    near_forces<T, false>(C, W, N, L, st, near, fx, fy, rec);
+    near_forces<T, false>(C, W, N, L, st, near, fx, fy, rec, true);
     const int listed = near < K ? near : K;  // every listed agent touches
     bad += rec.n != listed || rec.slow != (near > K || listed > NEAR_TOUCH);
     for (int e = 0; e < listed && e < NEAR_TOUCH; ++e)
