@@ -6,7 +6,7 @@
 // sum per tile on the device and, by its own store, in pinned host memory, so the host has the
 // edge count after one launch and one wait.  No prefix of single agents goes through memory: a
 // workgroup of k_edge_fill adds the tiles before its own, the counts before it in its tile, and
-// scans its 512 counts, all from reads that wait for nothing else; a row of up to four
+// scans its counts, 512 at a time, from reads that wait for nothing else; a row of up to four
 // neighbours is one 16-byte read.
 //
 // What bounds it: the wait, the launches and the gaps between them, then one line of the lists
@@ -26,7 +26,7 @@ int set_error(const char *msg);  // swarp_hip.hip: the message swarp_last_error(
 namespace {
 
 constexpr int EDGE_BLOCK = 256;                    // threads of a workgroup
-constexpr int EDGE_PART = 2 * EDGE_BLOCK;          // agents of a workgroup of k_edge_fill
+constexpr int EDGE_PART = 2 * EDGE_BLOCK;          // agents k_edge_fill scans at a time
 constexpr int64_t EDGE_TILE = 2048, EDGE_TILES = 1024;
 
 // Agents per tile (a multiple of EDGE_TILE) and how many tiles there are.
@@ -97,37 +97,58 @@ __device__ __forceinline__ void edges_of(int64_t i, int64_t e, int32_t A, int32_
     }
 }
 
+// A workgroup takes per / EDGE_TILE parts of EDGE_PART agents, a quarter of a tile whatever its
+// size, so that what it reads again (the counts before it in its tile, the tiles before) stays
+// below the counts themselves: of 64 M agents, 0.3 edges an agent, the graph took 1250 us with one
+// part a workgroup (and 1037 us with a library's prefix sum), now 600.  ONE: one part, up to 2 M
+// agents, compiled without the loop (1.0 M agents, count and fill 26.0 us, looping 27.5).
+template <bool ONE>
 __global__ __launch_bounds__(EDGE_BLOCK) void k_edge_fill(int64_t n, int64_t per, int32_t A,
                                                           int32_t K, const int32_t *idx,
                                                           const int32_t *cnt, const int64_t *sums,
                                                           int64_t n_edges, int64_t *out)
 {
     __shared__ int64_t before[EDGE_BLOCK / 64];
-    __shared__ int32_t wsum[EDGE_BLOCK / 64];
+    __shared__ int32_t wsum[2][EDGE_BLOCK / 64];  // by turns: one barrier a part
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int64_t i0 = (int64_t)blockIdx.x * EDGE_PART, tile = i0 / per;
-    const int64_t i = i0 + 2 * (int)threadIdx.x;
-    const int32_t c0 = i < n ? slots_of(cnt[i], K) : 0;
-    const int32_t c1 = i + 1 < n ? slots_of(cnt[i + 1], K) : 0;
-    int64_t b = share_of(cnt, tile * per, i0, K);
-    for (int64_t t = threadIdx.x; t < tile; t += EDGE_BLOCK) b += sums[t];
-    for (int d = 32; d > 0; d >>= 1) b += __shfl_down(b, d, 64);
-    int32_t v = c0 + c1;
-    for (int d = 1; d < 64; d <<= 1) {
-        const int32_t y = __shfl_up(v, d, 64);
-        if (lane >= d) v += y;
-    }
-    if (lane == 0) before[wv] = b;
-    if (lane == 63) wsum[wv] = v;
-    __syncthreads();
-    int64_t o = v - c0 - c1;
-    for (int w = 0; w < EDGE_BLOCK / 64; ++w) o += before[w] + (w < wv ? wsum[w] : 0);
-    if (i >= n) return;
+    const int64_t parts = ONE ? 1 : per / EDGE_TILE;
+    const int64_t start = (int64_t)blockIdx.x * parts * EDGE_PART, tile = start / per;
     const bool rows16 = (K & 3) == 0 && ((uintptr_t)idx & 15u) == 0;
-    const int64_t e0 = i0 / A;  // one 64-bit division per workgroup
-    const uint32_t r = (uint32_t)(i - e0 * A);
-    edges_of(i, e0 + r / (uint32_t)A, A, K, c0, idx, rows16, o, n_edges, out);
-    edges_of(i + 1, e0 + (r + 1) / (uint32_t)A, A, K, c1, idx, rows16, o + c0, n_edges, out);
+    int64_t base = 0;  // edges before the part
+    for (int64_t p = 0; p < parts; ++p) {
+        const int64_t i0 = start + p * EDGE_PART;
+        if (i0 >= n) return;
+        const int64_t i = i0 + 2 * (int)threadIdx.x;
+        const int32_t c0 = i < n ? slots_of(cnt[i], K) : 0;
+        const int32_t c1 = i + 1 < n ? slots_of(cnt[i + 1], K) : 0;
+        int32_t *const ws = wsum[p & 1];
+        if (p == 0) {
+            int64_t b = share_of(cnt, tile * per, start, K);
+            for (int64_t t = threadIdx.x; t < tile; t += EDGE_BLOCK) b += sums[t];
+            for (int d = 32; d > 0; d >>= 1) b += __shfl_down(b, d, 64);
+            if (lane == 0) before[wv] = b;
+        }
+        int32_t v = c0 + c1;
+        for (int d = 1; d < 64; d <<= 1) {
+            const int32_t y = __shfl_up(v, d, 64);
+            if (lane >= d) v += y;
+        }
+        if (lane == 63) ws[wv] = v;
+        __syncthreads();
+        if (p == 0)
+            for (int w = 0; w < EDGE_BLOCK / 64; ++w) base += before[w];
+        int64_t o = base + v - c0 - c1;
+        for (int w = 0; w < EDGE_BLOCK / 64; ++w) {
+            o += w < wv ? ws[w] : 0;
+            base += ws[w];
+        }
+        if (i < n) {
+            const int64_t e0 = i0 / A;  // one 64-bit division per part
+            const uint32_t r = (uint32_t)(i - e0 * A);
+            edges_of(i, e0 + r / (uint32_t)A, A, K, c0, idx, rows16, o, n_edges, out);
+            edges_of(i + 1, e0 + (r + 1) / (uint32_t)A, A, K, c1, idx, rows16, o + c0, n_edges, out);
+        }
+    }
 }
 
 int fail(const char *msg) { return swarp::set_error(msg); }
@@ -177,11 +198,16 @@ int swarp_edge_fill(int32_t n_envs, int32_t n_agents, int32_t max_neighbors, con
     if (n_edges == 0) return 0;
     if (!idx || !cnt || !sums || !edge_index) return fail("pointer arguments must be set");
     const int64_t n = (int64_t)n_envs * n_agents;
-    const int64_t blocks = (n + EDGE_PART - 1) / EDGE_PART;
-    if (blocks > 0x7fffffff) return fail("n_envs * n_agents is too large");
-    hipLaunchKernelGGL(k_edge_fill, dim3((unsigned)blocks), dim3(EDGE_BLOCK), 0,
-                       (hipStream_t)stream, n, edge_per(n), n_agents, max_neighbors, idx, cnt, sums,
-                       n_edges, edge_index);
+    const int64_t agents = edge_per(n) / EDGE_TILE * EDGE_PART;  // of a workgroup
+    const int64_t blocks = (n + agents - 1) / agents;           // (at most 4 EDGE_TILES)
+    const dim3 g((unsigned)blocks), b(EDGE_BLOCK);
+    hipStream_t st = (hipStream_t)stream;
+    if (agents == EDGE_PART)
+        hipLaunchKernelGGL((k_edge_fill<true>), g, b, 0, st, n, edge_per(n), n_agents, max_neighbors,
+                           idx, cnt, sums, n_edges, edge_index);
+    else
+        hipLaunchKernelGGL((k_edge_fill<false>), g, b, 0, st, n, edge_per(n), n_agents,
+                           max_neighbors, idx, cnt, sums, n_edges, edge_index);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(hipGetErrorString(e));
     return 0;

@@ -47,6 +47,15 @@ def test_edges_match_the_lists(E, A, K, fill):
     assert torch.equal(got, ref)
 
 
+@pytest.mark.parametrize("E,A,K,fill", [
+    (2100, 1000, 2, 0.5),   # just above 1024 tiles of 2048: two parts a workgroup
+    (6001, 701, 3, 0.3),    # three, a ragged end
+    (4100, 1023, 1, 1.0),   # a last workgroup with one agent of its second part
+])
+def test_more_agents_than_single_part_workgroups(E, A, K, fill):
+    test_edges_match_the_lists(E, A, K, fill)
+
+
 def test_no_edges_and_another_stream():
     g, _ = _lists(5, 300, 4, 1, 0.0)
     assert g.edge_index().shape == (2, 0)
