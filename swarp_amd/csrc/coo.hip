@@ -180,7 +180,11 @@ int swarp_edge_count(int32_t n_envs, int32_t n_agents, int32_t max_neighbors, co
     hipLaunchKernelGGL(k_edge_sums, dim3((unsigned)tiles), dim3(EDGE_BLOCK), 0, st, n, edge_per(n),
                        max_neighbors, cnt, sums, (int64_t *)dev);
     e = hipGetLastError();
-    if (e == hipSuccess) e = hipStreamSynchronize(st);
+    if (e == hipSuccess) {
+        e = hipStreamSynchronize(st);
+        // (reported here: not left for the next launch's check to find)
+        if (e != hipSuccess) (void)hipGetLastError();
+    }
     if (e != hipSuccess) return fail(hipGetErrorString(e));
     int64_t total = 0;
     for (int64_t t = 0; t < tiles; ++t) total += host_sums[t];

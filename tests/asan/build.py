@@ -82,6 +82,18 @@ def build(jobs: int = 8) -> Path:
     return EXE
 
 
+def build_coo() -> Path:
+    """tests/asan/_build/coo: coo.cpp with coo.hip under the sanitizers."""
+    OUT.mkdir(exist_ok=True)
+    stage()
+    exe = OUT / "coo"
+    r = subprocess.run(["g++", *FLAGS, f"-I{HERE / 'emu'}", f"-I{SRC}", "-x", "c++",
+                        str(HERE / "coo.cpp"), "-o", str(exe)], capture_output=True, text=True)
+    if r.returncode:
+        raise RuntimeError("coo build failed:\n" + (r.stdout + r.stderr)[-6000:])
+    return exe
+
+
 NEAR = ["-std=c++17", "-ffp-contract=off", "-pthread", "-w", f"-I{HERE / 'emu'}", f"-I{SRC}",
         str(HERE / "near.cpp")]
 CLANG = Path("/opt/rocm/llvm/bin/clang++")

@@ -91,7 +91,9 @@ struct Block {
 inline thread_local dim3 tIdx, bIdx;
 inline dim3 bDim, gDim;
 inline Block *block = nullptr;
-inline int last_error = 0;
+// The last error of a runtime call, which hipGetLastError hands out once, and an error for the
+// next hipStreamSynchronize to return (0: none).
+inline int last_error = 0, sync_error = 0;
 
 inline unsigned char *dyn_lds() { return block->lds->empty() ? nullptr : block->lds->data(); }
 
@@ -146,7 +148,24 @@ void launch(K kernel, dim3 grid, dim3 blk, size_t shm, A... args)
 #define gridDim (::emu::gDim)
 #define hipLaunchKernelGGL(K, G, B, SHM, ST, ...) ::emu::launch(K, dim3(G), dim3(B), (size_t)(SHM), __VA_ARGS__)
 
-inline hipError_t hipGetLastError() { return ::emu::last_error; }
+inline hipError_t hipGetLastError()
+{
+    const int e = ::emu::last_error;
+    ::emu::last_error = 0;
+    return e;
+}
+inline hipError_t hipStreamSynchronize(hipStream_t)
+{
+    const int e = ::emu::sync_error;
+    ::emu::sync_error = 0;
+    if (e) ::emu::last_error = e;
+    return e;
+}
+inline hipError_t hipHostGetDevicePointer(void **dev, void *host, unsigned)
+{
+    *dev = host;
+    return hipSuccess;
+}
 inline const char *hipGetErrorString(hipError_t) { return "emulated launch failure"; }
 
 inline void __syncthreads() { ::emu::block->bar.wait("block"); }
@@ -221,7 +240,6 @@ inline long long min(long long a, long long b) { return a < b ? a : b; }
 inline long long max(long long a, long long b) { return a > b ? a : b; }
 
 inline int atomicAdd(int *p, int v) { return __atomic_fetch_add(p, v, __ATOMIC_SEQ_CST); }
-inline int atomicExch(int *p, int v) { return __atomic_exchange_n(p, v, __ATOMIC_SEQ_CST); }
 
 inline float __builtin_amdgcn_sqrtf(float x) { return sqrtf(x); }
 inline double __builtin_amdgcn_rcp(double x) { return 1.0 / x; }
