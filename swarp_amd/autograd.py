@@ -167,6 +167,31 @@ def _empty_like_fields(stepper: Stepper, lead: tuple[int, ...], E: int, dev) -> 
     return [torch.empty(*lead, E, A, *_TAIL[k], device=dev, dtype=stepper.dtype) for k in range(nf)]
 
 
+#: From this size on a tape is taken only while it is at most an eighth of the device memory
+#: still free, so that a program whose graphs fill the card without tapes still runs: each
+#: retained tape leaves seven eighths of what it found.
+TAPE_CHECKED_FROM = 1 << 30
+
+
+def _tape_buffer(sizes, dev) -> torch.Tensor | None:
+    """A buffer of the first of ``sizes`` (bytes, largest first; 0: no tape) that memory is
+    there for, or None: a backward without its tape recomputes, with the same bits."""
+    for nb in sizes:
+        if not nb:
+            continue
+        if nb >= TAPE_CHECKED_FROM and not torch.cuda.is_current_stream_capturing():
+            # what the driver has free and what torch holds without using it
+            free = (torch.cuda.mem_get_info(dev)[0] + torch.cuda.memory_reserved(dev)
+                    - torch.cuda.memory_allocated(dev))
+            if nb > free // 8:
+                continue
+        try:
+            return torch.empty(nb, device=dev, dtype=torch.uint8)
+        except torch.OutOfMemoryError:
+            continue
+    return None
+
+
 class _RolloutFn(torch.autograd.Function):
     """T steps as one autograd node; outputs = final state fields, then the stacked
     trajectory fields of steps 0..T-2."""
@@ -188,8 +213,7 @@ class _RolloutFn(torch.autograd.Function):
         else:
             final, traj = bufs
         # the rollout tape lets the backward skip recomputing the substeps
-        nb = stepper.tape_bytes(E, actions_seq.shape[3], T)
-        tape = torch.empty(nb, device=dev, dtype=torch.uint8) if nb else None
+        tape = _tape_buffer((stepper.tape_bytes(E, actions_seq.shape[3], T),), dev)
         sink = KERNEL_EVENTS
         if sink is not None:
             e0 = _event(actions_seq)
@@ -257,10 +281,16 @@ class _RolloutFn(torch.autograd.Function):
         return (None, None, adj_act if need[2] else None, *adj0)
 
 
+def _check_ob_tape(stepper: Stepper, tape: torch.Tensor, E: int, ad: int, T: int) -> None:
+    sizes = stepper.ob_tape_sizes(E, ad, T)
+    check_extent(tape, tape.numel() if tape.numel() in sizes else sizes[0], "ob_tape", torch.uint8)
+
+
 def _launch_fwd_ob(stepper: Stepper, state0, ob0: torch.Tensor, actions_seq: torch.Tensor,
                    traj, final, ob_traj: torch.Tensor, tape: torch.Tensor | None = None) -> None:
     """One forward launch of a world with movable bodies (five state fields, nine with
-    drones); ``tape`` (uint8, ``Stepper.ob_tape_bytes`` long) also receives the body tape."""
+    drones); ``tape`` (uint8, one of ``Stepper.ob_tape_sizes`` long) also receives the body
+    tape."""
     T, E, _, ad = actions_seq.shape
     nf = _nfields(stepper)
     lib = _lib.load()
@@ -279,7 +309,7 @@ def _launch_fwd_ob(stepper: Stepper, state0, ob0: torch.Tensor, actions_seq: tor
             _stream(actions_seq),
         ))
         return
-    check_extent(tape, stepper.ob_tape_bytes(E, ad, T), "ob_tape", torch.uint8)
+    _check_ob_tape(stepper, tape, E, ad, T)
     _lib.check(lib.swarp_rollout_fwd_ob_tape(
         ctypes.byref(desc), T, ctypes.byref(s0), ob0.data_ptr(), actions_seq.data_ptr(),
         ctypes.byref(tr) if tr is not None else None, ctypes.byref(fin), ob_traj.data_ptr(),
@@ -305,9 +335,9 @@ class _RolloutObFn(torch.autograd.Function):
         final = _empty_like_fields(stepper, (), E, dev)
         traj = _empty_like_fields(stepper, (max(T - 1, 0),), E, dev)
         ob_traj = torch.empty((T,) + tuple(ob0.shape), device=dev, dtype=ob0.dtype)
-        # the body tape lets the backward skip evaluating the body pass again
-        nb = stepper.ob_tape_bytes(E, actions_seq.shape[3], T)
-        tape = torch.empty(nb, device=dev, dtype=torch.uint8) if nb else None
+        # the body tape lets the backward skip evaluating the body pass and the forces again, or,
+        # where memory is short, its records alone the body pass
+        tape = _tape_buffer(stepper.ob_tape_sizes(E, actions_seq.shape[3], T), dev)
         sink = KERNEL_EVENTS
         if sink is not None:
             e0 = _event(actions_seq)
@@ -368,7 +398,7 @@ class _RolloutObFn(torch.autograd.Function):
         if tape is None:
             _lib.check(lib.swarp_rollout_bwd_ob(*args, _stream(actions_seq)))
         else:
-            check_extent(tape, stepper.ob_tape_bytes(E, ad, T), "ob_tape", torch.uint8)
+            _check_ob_tape(stepper, tape, E, ad, T)
             _lib.check(lib.swarp_rollout_bwd_ob_tape(*args, tape.data_ptr(), tape.numel(),
                                                      _stream(actions_seq)))
         if sink is not None:

@@ -122,10 +122,12 @@ class Stepper:
         #: route eligible fleets to the specialised kernels (set False to force the
         #: generic ones; both give bit-identical results)
         self.use_specialised = True
-        #: grad rollouts on the specialised kernels keep a tape of the substep
-        #: intermediates, grad rollouts with movable bodies one of the body pass, so that
-        #: the backward does not recompute them (set False to recompute; both give
-        #: bit-identical results)
+        #: grad rollouts keep a tape of the substep intermediates, grad rollouts with movable
+        #: bodies one of the body pass and of what the agents felt, so that the backward does
+        #: not recompute them (set False to recompute; both give bit-identical results).  A
+        #: retained graph holds its tape: ``tape_bytes`` / ``ob_tape_sizes`` bytes, up to
+        #: 16 GiB for swarms and bodies.  Where memory is short it is left out
+        #: (``autograd._tape_buffer``)
         self.use_tape = True
         #: route fleets whose features a compiled profile covers (2-D fleets with
         #: obstacles and walls under Euler, drone fleets, holonomic fleets pushing movable
@@ -430,6 +432,16 @@ class Stepper:
                                                        ctypes.byref(c)))
             n = self._tape_sizes[key] = int(c.value)
         return n
+
+    def ob_tape_sizes(self, n_envs: int, act_dim: int, T: int) -> tuple[int, ...]:
+        """The sizes a body tape may have, largest first: the whole tape (``ob_tape_bytes``)
+        and the body records alone; (0,) where no tape is kept."""
+        full = self.ob_tape_bytes(n_envs, act_dim, T)
+        if not full:
+            return (0,)
+        item = 8 if self.dtype == torch.float64 else 4
+        records = T * self.substeps * n_envs * self.n_body_roots * 12 * item
+        return (full, records) if records < full else (full,)
 
     def grid(self, n_envs: int) -> NeighborGrid:
         g = self._grids.get(n_envs)
