@@ -217,6 +217,33 @@ int run_case(const Case &c)
         rc = swarp_rollout_bwd_ob(&d, nT, &s0, ob0, act, nT > 1 ? &traj : nullptr, obt,
                                   nT > 1 ? &atr : nullptr, &afin, aobt, &a0, aob0, aact, nullptr);
         if (rc) return fprintf(stderr, "%s bwd_ob: %s\n", c.name, swarp_last_error()), 1;
+        // the taped pair, with the whole tape and with the body records alone: the same bits (wider
+        // envs leave the tape unused)
+        uint64_t full = 0;
+        rc = swarp_ob_tape_bytes(&d, nT, 1, &full);
+        if (rc) return fprintf(stderr, "%s ob_tape_bytes: %s\n", c.name, swarp_last_error()), 1;
+        const uint64_t records = (uint64_t)nT * c.S * E * 12 * sizeof(T);
+        const std::vector<T> want_act(aact, aact + (size_t)nT * EA * ad);
+        const std::vector<T> want_ob(aob0, aob0 + (size_t)E * NW);
+        const T *a0p = (const T *)a0.pos;
+        const std::vector<T> want_pos(a0p, a0p + EA * 2);
+        for (uint64_t tb : {full, records}) {
+            if (A > 64) break;
+            void *tape = make<unsigned char>(tb, own);
+            rc = swarp_rollout_fwd_ob_tape(&d, nT, &s0, ob0, act, nT > 1 ? &traj : nullptr, &fin, obt,
+                                           tape, tb, nullptr);
+            if (rc) return fprintf(stderr, "%s fwd_ob_tape: %s\n", c.name, swarp_last_error()), 1;
+            rc = swarp_rollout_bwd_ob_tape(&d, nT, &s0, ob0, act, nT > 1 ? &traj : nullptr, obt,
+                                           nT > 1 ? &atr : nullptr, &afin, aobt, &a0, aob0, aact, tape,
+                                           tb, nullptr);
+            if (rc) return fprintf(stderr, "%s bwd_ob_tape: %s\n", c.name, swarp_last_error()), 1;
+            for (size_t q = 0; q < want_act.size(); ++q)
+                if (aact[q] != want_act[q]) return fprintf(stderr, "%s: taped d/d actions\n", c.name), 1;
+            for (size_t q = 0; q < want_ob.size(); ++q)
+                if (aob0[q] != want_ob[q]) return fprintf(stderr, "%s: taped d/d ob0\n", c.name), 1;
+            for (size_t q = 0; q < want_pos.size(); ++q)
+                if (a0p[q] != want_pos[q]) return fprintf(stderr, "%s: taped d/d pos\n", c.name), 1;
+        }
     } else if (c.wheel) {
         rc = swarp_rollout_fwd(&d, nT, &s0, act, nT > 1 ? &traj : nullptr, &fin, nullptr);
         if (rc) return fprintf(stderr, "%s fwd: %s\n", c.name, swarp_last_error()), 1;
@@ -253,6 +280,21 @@ int run_case(const Case &c)
     int32_t *idx = make<int32_t>(EA * c.K, own), *cnt = make<int32_t>(EA, own), *tru = make<int32_t>(EA, own);
     rc = swarp_neighbors(&d, s0.pos, idx, cnt, tru, nullptr);
     if (rc) return fprintf(stderr, "%s neighbors: %s\n", c.name, swarp_last_error()), 1;
+    // and rows of other lengths: whole and packed ones, not whole 16-byte pieces, more slots than
+    // agents
+    for (int K : {3, 16, 17, 20, 35, 80}) {
+        if (A > 70) break;  // (the emulation of many waves is slow)
+        d.max_neighbors = K;
+        int32_t *rows = make<int32_t>(EA * K, own);
+        rc = swarp_neighbors(&d, s0.pos, rows, cnt, nullptr, nullptr);
+        if (rc) return fprintf(stderr, "%s neighbors K=%d: %s\n", c.name, K, swarp_last_error()), 1;
+        for (size_t i = 0; i < EA; ++i)
+            for (int k = 0; k < K; ++k) {
+                const int j = rows[i * K + k];
+                if (cnt[i] > K || j < 0 || j >= A || (k >= cnt[i] && j != 0))
+                    return fprintf(stderr, "%s neighbors K=%d: row %zu\n", c.name, K, i), 1;
+            }
+    }
     for (auto p : own) free(p);
     printf("%-28s ok\n", c.name);
     fflush(stdout);
@@ -284,6 +326,8 @@ int main(int argc, char **argv)
         {"boxes f32",            7, 16, 3, 2, 8, 2, 3, false, true,  true,  false, false, false, 1},
         {"holonomic f64 A=5",   11, 5, 4, 3, 4, 2, 0, false, false, true,  false, false, false, 0},
         {"wide f32 A=100",       2, 100, 3, 2, 12, 2, 3, false, false, true,  false, false, false, 1},
+        {"wide per-env f32 A=100", 2, 100, 3, 2, 12, 2, 0, false, false, true, false, false, false, 0, true},
+        {"wide f32 A=70 one step", 2, 70, 1, 1, 8, 2, 0, false, false, true, false, false, false, 0},
         {"wide grid f32 A=70",   2, 70, 3, 2, 8, 2, 0, false, false, true,  false, false, true,  0},
         {"wide bodies f32 A=100", 2, 100, 3, 2, 12, 2, 5, false, false, true, true, false, false, 0},
         {"wide bodies grid f32 A=70", 2, 70, 3, 2, 8, 2, 5, false, false, true, true, false, true, 0},

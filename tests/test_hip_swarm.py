@@ -63,7 +63,7 @@ def test_grid_lists_in_crowded_cells(A, spread):
 
 @pytest.mark.parametrize("E,A,T,S,half,kw", [
     (5, 65, 6, 4, 2.2, {}),                               # just past a wavefront, sparse
-    (3, 256, 5, 3, 4.0, {}),                              # every slot of the small hash in use
+    (3, 256, 5, 3, 4.0, {}),                              # four waves, sparse
     (2, 200, 4, 4, 0.9, {}),                              # candidate lists overflow: full traversal
     (3, 130, 5, 2, 1.6, dict(max_neighbors=3)),           # lists truncated among few candidates
     (2, 90, 5, 2, 0.8, dict(neighbor_radius=0.3, max_neighbors=5)),
@@ -77,7 +77,7 @@ def test_grid_lists_in_crowded_cells(A, spread):
     (1, 3584, 2, 2, 12.0, dict(neighbor_method="brute")),  # the largest env: the shortest lists
     (2, 100, 4, 2, 1.6, dict(f64=True)),
     (1, 2048, 2, 2, 10.0, dict(f64=True, neighbor_method="brute")),
-    (3, 80, 5, 4, 1.5, dict(shift=40000.0)),              # beyond the hash's certain range
+    (3, 80, 5, 4, 1.5, dict(shift=40000.0)),              # far from the origin: coarse positions
     (3, 96, 5, 4, 2.0, dict(fast=6.0)),                   # agents outrun the skin
     (3, 96, 5, 2, 1.1, dict(mixed=True)),                 # diff-drive and bicycle
 ])
