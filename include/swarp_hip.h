@@ -179,7 +179,7 @@ int swarp_rollout_bwd(const swarp_desc_t *desc, int32_t T, const swarp_state_t *
  * (StepBuffers / make_buffers, swarp/core/stepper.py:55-63, 642-678).
  * Writes in *bytes the tape size of a T-step rollout of this configuration; 0 when the
  * configuration keeps no tape, in which case the _tape entry points behave as the plain
- * ones.  Three kinds of configuration keep one: fleets on the specialised holonomic-velocity
+ * ones.  Four kinds of configuration keep one: fleets on the specialised holonomic-velocity
  * kernels with substeps <= 4 and contacts or walls (the records above), and float32 2-D
  * fleets among static obstacles whose forward runs the obstacle pass on a wave of its own
  * (at most 256 / (envs per 64 lanes) obstacles, no box agents, wheel contacts or drones):
@@ -188,11 +188,15 @@ int swarp_rollout_bwd(const swarp_desc_t *desc, int32_t T, const swarp_state_t *
  * 32 agents), which the backward reads instead of evaluating the forces and scanning, and
  * for at most 32 obstacles each substep's per-agent mask of the obstacles in contact,
  * w T S E A bytes more (w = 1, 2 or 4 for up to 8, 16 or 32 obstacles; each part rounded
- * up to 256), so that the backward reverses only those; and the other fleets without box
- * agents or wheel contacts that have contacts, walls or obstacles (drones among them):
- * each substep's total force and neighbour mask as above, no contact masks.  The taped
- * backward gives the
- * untaped one's values; a gradient that is zero may differ in the sign of that zero. */
+ * up to 256), so that the backward reverses only those; the other fleets of up to 64 agents per
+ * env with index-ordered lists, without box agents or wheel contacts, that have contacts, walls
+ * or obstacles (drones and RK4 fleets among them): each substep's total force and neighbour mask
+ * as above, no contact masks; and the same fleets in envs of more than 64 agents or with
+ * grid-ordered lists: each substep's total force, 2 T S E A scalars, and with contacts the
+ * agents each agent touched, 16 T S E A bytes (each part rounded up to 256).  This last kind is
+ * kept up to 16 GiB: the size of a longer rollout is 0, so sizes are asked for the T that is run.
+ * The taped backward gives the untaped one's values; a gradient that is zero may differ in the
+ * sign of that zero. */
 int swarp_tape_bytes(const swarp_desc_t *desc, int32_t T, uint64_t *bytes);
 
 /* swarp_rollout_fwd that also writes the tape (`tape_bytes` must be
@@ -264,13 +268,18 @@ int swarp_rollout_bwd_ob_check(const swarp_desc_t *desc);
  * forward so that the backward's recompute of each step reads it instead of evaluating
  * the pass again; and, up to 64 agents per env with index-ordered lists, behind those
  * records what the agents felt (forces and touching agents of the few that feel any, the
- * shapes touched), read instead of evaluating their forces again.  Bodies are counted in root order (the obstacle indices o with body[o] = o and kind[o] = 1);
- * a tape may hold the first n_bodies of them, and the backward evaluates the others.
+ * shapes touched), read instead of evaluating their forces again.  Bodies are counted in root
+ * order (the obstacle indices o with body[o] = o and kind[o] = 1); a tape may hold the first
+ * n_bodies of them, and the backward evaluates the others.
  * No counterpart in the reference: its body pass runs on untaped steps and is not
  * differentiated (swarp/core/stepper.py:952-991).
  * Writes in *bytes the size of the tape of a T-step rollout holding n_bodies bodies
- * (1 <= n_bodies <= n_obstacles).  A tape of T * substeps * n_envs * n_bodies * 12 scalars
- * holds the body records alone and is taken too (a slower backward, the same results). */
+ * (1 <= n_bodies <= n_obstacles): T * substeps * n_envs * n_bodies * 12 scalars of records and,
+ * where what the agents felt is kept, T * substeps * waves * (64 + 64 (2 scalars + 4 bytes, 8
+ * above 32 agents)) bytes behind them -- a wave holds 64 / (n_agents rounded up to a power of
+ * two) envs.  That part is reserved for agents that all feel something (1088 bytes a wave, of
+ * which a sparse env moves some 130) and left out above 16 GiB.  A tape of the records' size
+ * alone is taken too (a slower backward, the same results). */
 int swarp_ob_tape_bytes(const swarp_desc_t *desc, int32_t T, int32_t n_bodies, uint64_t *bytes);
 
 /* swarp_rollout_fwd_ob that also writes the body tape (device memory owned by the caller;
